@@ -64,6 +64,11 @@ class SolverInfo(ctypes.Structure):
                 ("split_couplings", I64 * 2)]
 
 
+class BlockInfo(ctypes.Structure):
+    _fields_ = [("rows", I64), ("bytes", ctypes.c_uint64), ("level_bytes", ctypes.c_uint64 * 2),
+                ("tail_bytes", ctypes.c_uint64 * 2), ("level_launches", I64 * 2), ("tail_runs", I64 * 2)]
+
+
 _SIGS = {
     "apx_last_error": ([], ctypes.c_char_p),
     "apx_options_default": ([P], None),
@@ -95,6 +100,7 @@ _SIGS = {
     "apx_solver_create_with_factor": ([I64, P, P, P, P, P, P], ctypes.c_int),
     "apx_solver_destroy": ([P], None),
     "apx_solver_info_get": ([P, P], ctypes.c_int),
+    "apx_solver_block_get": ([P, P], ctypes.c_int),
     "apx_solver_solve": ([P, P, P, P, F64, I32, P, P], ctypes.c_int),
     "apx_solver_solve_host": ([P, P, P, P, F64, I32, P], ctypes.c_int),
     "apx_solver_apply": ([P, P, P, P], ctypes.c_int),
@@ -383,6 +389,11 @@ class Solver:
         _check(load_library().apx_solver_info_get(self._h, ctypes.byref(inf)))
         self.info = {k: (list(v) if isinstance(v, ctypes.Array) else v)
                      for k, v in ((k, getattr(inf, k)) for k, _ in SolverInfo._fields_)}
+        blk = BlockInfo()
+        _check(load_library().apx_solver_block_get(self._h, ctypes.byref(blk)))
+        # The trailing block of an application and the launches outside it.
+        self.info["block"] = {k: (list(v) if isinstance(v, ctypes.Array) else v)
+                              for k, v in ((k, getattr(blk, k)) for k, _ in BlockInfo._fields_)}
 
     def close(self):
         if getattr(self, "_h", None) and _lib is not None:

@@ -255,6 +255,22 @@ apx_status apx_solver_create_with_factor(int64_t n, const int64_t* colptr, const
 
 void apx_solver_destroy(apx_solver_t s) { delete s; }
 
+apx_status apx_solver_block_get(apx_solver_t s, apx_block_info* info) {
+    return guarded([&] {
+        need(s, "solver");
+        need(info, "info");
+        const solver_stats& st = s->s->stats();
+        info->rows = st.trail_rows;
+        info->bytes = st.trail_bytes;
+        for (int k = 0; k < 2; ++k) {
+            info->level_bytes[k] = st.solve_level_bytes[k];
+            info->tail_bytes[k] = st.solve_tail_bytes[k];
+            info->level_launches[k] = st.solve_level_launches[k];
+            info->tail_runs[k] = st.solve_tail_runs[k];
+        }
+    });
+}
+
 apx_status apx_solver_info_get(apx_solver_t s, apx_solver_info* info) {
     return guarded([&] {
         need(s, "solver");

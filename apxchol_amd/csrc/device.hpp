@@ -43,6 +43,7 @@ struct sweep_desc {
     const std::uint32_t* batch_pos = nullptr;  // nb+1
     const std::uint64_t* batch_mask = nullptr; // nb
     int nb = 0;
+    int b_first = 0;                        // dataflow launch: its first batch (the launch ends at nb)
     int chunk = 1;                          // batches claimed per ticket (dataflow schedule)
     int* ctrl = nullptr;                    // 2 ints: ticket, finished waves (zero between sweeps)
 };
@@ -158,6 +159,29 @@ struct tail_desc {
 struct alignas(8) lane_rec {
     std::int32_t row;    // the lane's row, or -1 for an idle lane
     std::uint32_t info;  // log2 G | sub << 3 | nvalid << 9
+};
+
+// The trailing block: the last n rows of the factor (storage rows [first,
+// first + n)), applied through its explicit inverse S = T^-T W T^-1 (see
+// kernels/trail.hip). The coupling to the rows before it comes as lane batches
+// (rec.row: row of the block; ent.idx: storage row) and a list of long rows
+// {block row, first entry, entries, 0} in the factor's own forward lists.
+inline constexpr int kTrailThreads = 1024;    // workgroup of the product
+inline constexpr int kTrailLine = 128;        // bytes of a row of S one workgroup of the product owns
+inline constexpr int kCoupleThreads = 512;    // workgroup of the coupling launch
+inline constexpr int kTrailMaxRows = 8192;    // c fits the LDS of a workgroup (64 KB in fp64)
+struct trail_desc {
+    int first = 0;
+    int n = 0;                       // rows of the block; 0: no block
+    int ld = 0;                      // row pitch of s, a multiple of 64
+    int chunk = 0;                   // k range of one partial sum, a multiple of 4; s holds
+                                     // kTrailThreads / (kTrailLine / value bytes) * chunk rows
+    const void* s = nullptr;         // S (fp64 or fp32), zero past n in both directions
+    const lane_rec* rec = nullptr;
+    const entry32* ent = nullptr;
+    int npack = 0;                   // lane batches
+    int nlong = 0;
+    const int4* longrow = nullptr;
 };
 
 // Per (tail batch, lane), written by the coupling kernel before a run: the

@@ -20,6 +20,7 @@
 
 #include "../device.hpp"
 #include "../kernels/launch.hpp"
+#include "trail.hpp"
 
 namespace apxchol_amd {
 
@@ -523,6 +524,9 @@ struct gpu_solver::device_state {
     int lanes = 8;
     dbuf r, x, p, ap, rp, y, z, xout;
     dbuf relabel;   // factor position -> storage position (empty: identity)
+    // The trailing block (t.n == 0: none), its product's input and layouts.
+    trail_desc trail;
+    dbuf tr_s, tr_c, tr_rec, tr_ent, tr_long;
     dbuf part, st, st_apply, ctrl, err;
     pcg_state* host_st = nullptr;
     int* host_err = nullptr;
@@ -547,7 +551,7 @@ struct gpu_solver::device_state {
     struct block_bufs {
         int kp = 0;
         std::map<int, std::unique_ptr<block_tables>> tables;   // per block width
-        dbuf r, x, p, ap, y, z, st, bs, part;
+        dbuf r, x, p, ap, y, z, c, st, bs, part;
         pcg_state* host_st = nullptr;
         batch_state* host_bs = nullptr;
         hipGraph_t graph = nullptr;
@@ -928,6 +932,15 @@ void gpu_solver::setup(const csc_view& L) {
     const int lane_max = opts_.lane_batches < 0 ? 0
                          : opts_.lane_batches > 0 ? opts_.lane_batches
                                                   : env_int("APXCHOL_AMD_LANE_BATCHES", 4096);
+    // The trailing block starts at a level boundary that depends on the factor
+    // and the vector precision alone, so every schedule agrees on it
+    // (APXCHOL_AMD_TRAIL_ROWS: the longest run of last levels of at most that
+    // many rows; 0: no block).
+    const std::size_t L_all = d.f_levels.empty() ? 0 : d.f_levels.size() - 1;
+    int trail_max = -1;
+    if (const char* e = std::getenv("APXCHOL_AMD_TRAIL_ROWS"); e && *e) trail_max = std::max(0, std::atoi(e));
+    std::size_t cut = choose_trail_level(T_, d.prec == vec_prec::fp64 ? 8 : 4, d.f_levels, d.b_levels, trail_max);
+    if (cut < L_all && !build_trail(T_.level_ptr[cut])) cut = L_all;
     auto make_sched = [&](sweep_sched& sc, const batch_table& bt, bool backward, const std::vector<int>& lf,
                           dbuf& lf_dev, std::vector<int> (&seg)[8], dbuf* const (&tbuf)[6], std::vector<int>& level_lb,
                           dbuf& lrec, dbuf& lent, std::vector<int>& level_pos, std::vector<unsigned char>& level_diag) {
@@ -964,7 +977,12 @@ void gpu_solver::setup(const csc_view& L) {
             }
             return worst;
         };
+        // The trailing block's boundary in this direction; no run crosses it.
+        const int cl = backward ? L - static_cast<int>(cut) : static_cast<int>(cut);
+        sc.cut_level = cl;
+        sc.cut_batch = lf[cl];
         for (int l = 0; l < L;) {
+            if (l == cl) sc.cut_seg = static_cast<int>(seg[0].size());
             if (!small(l)) {
                 seg[0].push_back(l); seg[1].push_back(l + 1); seg[2].push_back(0);
                 seg[3].push_back(pos(l)); seg[4].push_back(pos(l + 1)); seg[5].push_back(-1); seg[6].push_back(1);
@@ -972,7 +990,7 @@ void gpu_solver::setup(const csc_view& L) {
                 continue;
             }
             int e = l;
-            while (e < L && small(e) && sweep_tail_fits(tail_prec, pos(e + 1) - pos(l), lf[e + 1] - lf[l], e + 1 - l) &&
+            while (e < L && (e == l || e != cl) && small(e) && sweep_tail_fits(tail_prec, pos(e + 1) - pos(l), lf[e + 1] - lf[l], e + 1 - l) &&
                    (e == l || tail_cut <= 0 || ovf_groups(e, pos(l)) < tail_cut))
                 ++e;
             if (e == l) ++e;   // a single small level always fits (rows < tail_rows <= cap)
@@ -987,6 +1005,7 @@ void gpu_solver::setup(const csc_view& L) {
             }
             l = e;
         }
+        if (cl == L) sc.cut_seg = static_cast<int>(seg[0].size());
         const std::size_t tb = static_cast<std::size_t>(tt.batches);
         if (tt.lane.size() != tb * kWave || tt.lane_recip.size() != tb * kWave ||
             tt.ent.size() != tb * kTailPairs * kWave || tt.ovf.size() != tb || tt.ovf_ent.size() % kWave != 0 ||
@@ -1021,6 +1040,7 @@ void gpu_solver::setup(const csc_view& L) {
                 static_cast<std::uint64_t>(std::max(env_flag("APXCHOL_AMD_COUPLE_SPLIT_MIN", 1 << 20), 0));
             for (std::size_t k = 1; k < seg[0].size(); ++k) {
                 if (!seg[2][k] || !seg[2][k - 1] || seg[3][k - 1] <= 0) continue;
+                if (static_cast<int>(k) == sc.cut_seg) continue;   // a launch may start here
                 const int ps = seg[3][k - 1];
                 std::uint64_t before = 0;
                 for (int t = seg[3][k]; t < seg[4][k]; ++t) {
@@ -1099,8 +1119,14 @@ void gpu_solver::setup(const csc_view& L) {
             for (std::size_t k = 0; k < seg[0].size(); ++k) {
                 const bool tail = sc.kind == 2 && seg[2][k];
                 for (int q = seg[0][k]; q < seg[1][k]; ++q) {
-                    if (tail) stats_.tail_bytes[di] += level_b(q);
-                    else { stats_.level_bytes[di] += level_b(q); ++stats_.level_launches[di]; }
+                    const std::uint64_t lb = level_b(q);
+                    const bool outside = cut == static_cast<std::size_t>(L) || (backward ? q >= cl : q < cl);
+                    if (tail) stats_.tail_bytes[di] += lb;
+                    else { stats_.level_bytes[di] += lb; ++stats_.level_launches[di]; }
+                    if (!outside) continue;
+                    if (tail) stats_.solve_tail_bytes[di] += lb;
+                    else { stats_.solve_level_bytes[di] += lb; ++stats_.solve_level_launches[di]; }
+                    if (tail && q == seg[0][k]) ++stats_.solve_tail_runs[di];
                 }
                 if (tail) ++stats_.tail_runs[di];
             }
@@ -1175,10 +1201,13 @@ void gpu_solver::setup(const csc_view& L) {
                           &d.op_val, &d.r, &d.x, &d.p, &d.ap, &d.rp, &d.y, &d.z, &d.xout, &d.f_lrec, &d.f_lent,
                           &d.b_lrec, &d.b_lent, &d.f_tlane, &d.f_tent, &d.f_tovf, &d.f_tovf_ent, &d.f_twalk,
                           &d.b_tlane, &d.b_tent, &d.b_tovf, &d.b_tovf_ent, &d.b_twalk, &d.f_tlane_r, &d.b_tlane_r,
-                          &d.tail_val, &d.relabel, &d.sell_soff,
+                          &d.tail_val, &d.relabel, &d.tr_s, &d.tr_c, &d.tr_rec, &d.tr_ent, &d.tr_long, &d.sell_soff,
                           &d.sell_idx, &d.sell_val, &d.sell_map, &d.sell_long})
         bytes += b->bytes();
     stats_.device_bytes = bytes;
+    // What one application runs outside the trailing block.
+    stats_.trail_rows = d.trail.n;
+    stats_.trail_bytes = d.trail.n > 0 ? static_cast<std::uint64_t>(d.trail.n) * d.trail.n * (d.prec == vec_prec::fp64 ? 8 : 4) : 0;
 
     if (!opts_.keep_factor_values) {
         std::vector<node_t>().swap(F_.inner);
@@ -1188,6 +1217,72 @@ void gpu_solver::setup(const csc_view& L) {
     // Everything but the operator build is the SpTRSV side (preparation,
     // layouts, uploads of both).
     setup_times_.sptrsv_setup_ms = ms_since(t_setup) - setup_times_.pcg_setup_ms;
+}
+
+bool gpu_solver::build_trail(std::uint32_t first) {
+    auto& d = *dev_;
+    const int n = static_cast<int>(T_.m - first);
+    const std::size_t vsz = d.prec == vec_prec::fp64 ? sizeof(double) : sizeof(float);
+    const int np = (n + kWave - 1) / kWave * kWave;
+    const int chunks = trail_chunks(d.prec);
+    trail_desc t;
+    t.first = static_cast<int>(first);
+    t.n = n;
+    t.ld = np;
+    t.chunk = ((n + chunks - 1) / chunks + 3) / 4 * 4;
+    const std::size_t values = static_cast<std::size_t>(chunks) * t.chunk * np;
+    dbuf a(static_cast<std::size_t>(np) * np * sizeof(double)), x(a.bytes()), bad(sizeof(double));
+    d.tr_s.alloc(values * vsz);
+    launch_trail_setup(d.fwd, T_.fp16 ? d.inv_scale.as<float>() : nullptr, d.prec, T_.fp16, t.first, n, np,
+                       a.as<double>(), x.as<double>(), d.tr_s.get(), values, np, bad.as<int>(), nullptr);
+    int flag = 0;
+    hip_check(hipMemcpy(&flag, bad.get(), sizeof flag, hipMemcpyDeviceToHost), "trailing block");
+    if (flag != 0) {   // an inverse outside the vectors' range: the levels are walked
+        d.tr_s.alloc(0);
+        return false;
+    }
+    const trail_couple_tables ct = build_trail_couple(T_, first);
+    d.tr_rec.upload(ct.rec);
+    d.tr_ent.upload(ct.ent);
+    d.tr_long.upload(ct.longrow);
+    d.tr_c.alloc(static_cast<std::size_t>(n) * sizeof(double));
+    t.s = d.tr_s.get();
+    t.rec = d.tr_rec.as<lane_rec>();
+    t.ent = d.tr_ent.as<entry32>();
+    t.npack = ct.batches;
+    t.nlong = static_cast<int>(ct.longrow.size());
+    t.longrow = d.tr_long.as<int4>();
+    d.trail = t;
+    return true;
+}
+
+// One preconditioner application without its permutations: z = L^-T W L^-1 r
+// in storage order.
+void gpu_solver::enqueue_pair(const double* r, const pcg_state* st, int step, hipStream_t s) const {
+    auto& d = *dev_;
+    timer& tm = *timer_;
+    int* err = d.err.as<int>();
+    const sweep_part rows = d.trail.n > 0 ? sweep_part::outside_block : sweep_part::whole;
+    tm.time(0, step, s, [&] {
+        launch_sweep(d.fwd, d.prec, d.fp16, r, d.y.get(), st, err, d.f_sched, s, tm.hook(step), rows);
+        if (d.trail.n > 0)
+            launch_trail(d.trail, d.fwd, d.prec, d.fp16, r, d.y.get(), d.tr_c.as<double>(), d.z.get(), st, s, tm.hook(step));
+    });
+    tm.time(1, step, s, [&] {
+        launch_sweep(d.bck, d.prec, d.fp16, d.y.get(), d.z.get(), st, err, d.b_sched, s, tm.hook(step), rows);
+    });
+}
+
+// The same for kp columns in the block buffers `which`.
+void gpu_solver::enqueue_pair_k(int kp, const pcg_state* st, const batch_state* bs, hipStream_t s, int which) const {
+    auto& d = *dev_;
+    auto& b = block_in(*dev_, which);
+    const auto& t = *b.tables.at(kp);
+    const sweep_part rows = d.trail.n > 0 ? sweep_part::outside_block : sweep_part::whole;
+    launch_sweep_k(d.fwd, d.prec, d.fp16, t.f, b.r.get(), b.y.get(), st, bs, s, rows);
+    if (d.trail.n > 0)
+        launch_trail_k(d.trail, d.fwd, d.prec, d.fp16, kp, b.r.as<double>(), b.y.get(), b.c.as<double>(), b.z.get(), st, bs, s);
+    launch_sweep_k(d.bck, d.prec, d.fp16, t.b, b.y.get(), b.z.get(), st, bs, s, rows);
 }
 
 void gpu_solver::check_sweep_error() const {
@@ -1208,18 +1303,12 @@ void gpu_solver::enqueue_precondition(bool first, int step, hipStream_t s) const
     const int m = static_cast<int>(T_.m);
     pcg_state* st = d.st.as<pcg_state>();
     double* part = d.part.as<double>();
-    int* err = d.err.as<int>();
     const vec_prec pr = d.prec;
     // The pending sentinels only for the dataflow schedule (the only one
     // that polls the outputs); the zero past the sweep rows of z always.
     void* sentinel_y = opts_.schedule == sweep_schedule::dataflow ? d.y.get() : nullptr;
     if (first) launch_fill_outputs(pr, n, m, sentinel_y, d.z.get(), st, s);
-    tm.time(0, step, s, [&] {
-        launch_sweep(d.fwd, pr, d.fp16, d.r.get(), d.y.get(), st, err, d.f_sched, s, tm.hook(step));
-    });
-    tm.time(1, step, s, [&] {
-        launch_sweep(d.bck, pr, d.fp16, d.y.get(), d.z.get(), st, err, d.b_sched, s, tm.hook(step));
-    });
+    enqueue_pair(d.r.as<double>(), st, step, s);
     tm.time(3, step, s, [&] {
         launch_dot_center(pr, n, d.r.as<double>(), d.z.get(), st, part, first, s);
         launch_update_p(pr, n, d.p.as<double>(), d.z.get(), st, first, s);
@@ -1397,6 +1486,7 @@ int gpu_solver::prepare_block(int k, int which) const {
     b.drop_graph();
     const std::size_t vb = static_cast<std::size_t>(std::max<std::int64_t>(n_, 1)) * kp * sizeof(double);
     b.r.alloc(vb); b.x.alloc(vb); b.p.alloc(vb); b.ap.alloc(vb); b.y.alloc(vb); b.z.alloc(vb);
+    b.c.alloc(static_cast<std::size_t>(dev_->trail.n) * kp * sizeof(double));
     b.st.alloc(static_cast<std::size_t>(kp) * sizeof(pcg_state));
     b.bs.alloc(sizeof(batch_state));
     // Partials: 2 values x kp columns per workgroup; the SpMM grid may round
@@ -1443,9 +1533,7 @@ void gpu_solver::apply_block(int k, const double* d_R, double* d_Z, bool center,
         launch_shift_from_sum_k(kp, st, true, s);
     }
     block_scheds(kp);
-    const auto& t = *b.tables.at(kp);
-    launch_sweep_k(d.fwd, d.prec, d.fp16, t.f, b.r.get(), b.y.get(), st, bs, s);
-    launch_sweep_k(d.bck, d.prec, d.fp16, t.b, b.y.get(), b.z.get(), st, bs, s);
+    enqueue_pair_k(kp, st, bs, s);
     if (center) launch_sum_cols_k(d.prec, n, kp, b.z.get(), st, part, s);
     launch_gather_k(d.prec, n, k, kp, d.perm.as<unsigned>(), b.z.get(), d_Z, st, center, s);
 }
@@ -1546,7 +1634,12 @@ const block_sched* gpu_solver::block_scheds(int kp, int which) const {
             const int block_tail_waves =
                 std::clamp(env_flag("APXCHOL_AMD_BLOCK_TAIL_WAVES", kTailWaves), 1, kBlockTailMaxWaves);
             const int nl = static_cast<int>(L);
+            block_sched& sc = backward ? t->b : t->f;
+            const int cl = (backward ? dev_->b_sched : dev_->f_sched).cut_level;
+            sc.cut_level = cl;
+            sc.cut_seg = 0;
             for (int l = 0; l < nl;) {
+                if (l == cl) sc.cut_seg = static_cast<int>(seg[0].size());
                 auto small = [&](int q) { return tails && lf[q + 1] - lf[q] <= block_tail_waves; };
                 if (!small(l)) {
                     seg[0].push_back(l); seg[1].push_back(l + 1); seg[2].push_back(0);
@@ -1554,7 +1647,7 @@ const block_sched* gpu_solver::block_scheds(int kp, int which) const {
                     continue;
                 }
                 int e = l;
-                while (e < nl && small(e) && lpos[e + 1] - lpos[l] <= cap) ++e;
+                while (e < nl && (e == l || e != cl) && small(e) && lpos[e + 1] - lpos[l] <= cap) ++e;
                 if (e == l) {   // one small level wider than the LDS: launch it
                     seg[0].push_back(l); seg[1].push_back(l + 1); seg[2].push_back(0);
                     ++l;
@@ -1563,7 +1656,7 @@ const block_sched* gpu_solver::block_scheds(int kp, int which) const {
                 seg[0].push_back(l); seg[1].push_back(e); seg[2].push_back(1);
                 l = e;
             }
-            block_sched& sc = backward ? t->b : t->f;
+            if (cl == nl) sc.cut_seg = static_cast<int>(seg[0].size());
             sc.kp = kp;
             sc.pos = dp.as<unsigned>();
             sc.mask = dm.as<unsigned long long>();
@@ -1611,9 +1704,7 @@ void gpu_solver::enqueue_precondition_k(bool first, int kp, hipStream_t s, int w
     pcg_state* st = b.st.as<pcg_state>();
     batch_state* bs = b.bs.as<batch_state>();
     block_scheds(kp, which);
-    const auto& t = *b.tables.at(kp);
-    launch_sweep_k(d.fwd, d.prec, d.fp16, t.f, b.r.get(), b.y.get(), st, bs, s);
-    launch_sweep_k(d.bck, d.prec, d.fp16, t.b, b.y.get(), b.z.get(), st, bs, s);
+    enqueue_pair_k(kp, st, bs, s, which);
     launch_dot_center_k(d.prec, n, kp, b.r.as<double>(), b.z.get(), st, bs, b.part.as<double>(), first, s);
     launch_update_p_k(d.prec, n, kp, b.p.as<double>(), b.z.get(), st, bs, first, s);
 }
@@ -1725,13 +1816,11 @@ gpu_solver::autotune_result gpu_solver::autotune(int max_block_width, hipStream_
             prepare_block(kp);
             block_scheds(kp);
             auto& b = d.blk;
-            const auto& t = *b.tables.at(kp);
             const std::size_t vb = static_cast<std::size_t>(n) * kp * sizeof(double);
             hip_check(hipMemsetAsync(b.r.get(), 0, vb, s), "memset");
             hip_check(hipMemsetAsync(b.y.get(), 0, vb, s), "memset");
             res.sweep_pair_us[k] = timed([&] {
-                launch_sweep_k(d.fwd, d.prec, d.fp16, t.f, b.r.get(), b.y.get(), nullptr, nullptr, s);
-                launch_sweep_k(d.bck, d.prec, d.fp16, t.b, b.y.get(), b.z.get(), nullptr, nullptr, s);
+                enqueue_pair_k(kp, nullptr, nullptr, s);
             }, 2);
             const double rate = kp / res.sweep_pair_us[k];
             if (rate > best_rate) { best_rate = rate; res.block_width = kp; }
@@ -1959,11 +2048,9 @@ void gpu_solver::apply_device(const double* d_r, double* d_z, hipStream_t s) con
     const bool center = !F_.sddm && (++apply_count_ % static_cast<std::uint64_t>(center_k_) == 0);
     pcg_state* st = d.st_apply.as<pcg_state>();
     double* part = d.part.as<double>();
-    int* err = d.err.as<int>();
     launch_sum_shift(n, d_r, st, part, center, s);
     launch_apply_scatter(d.prec, n, m, d.perm.as<unsigned>(), d_r, d.rp.as<double>(), d.y.get(), d.z.get(), s);
-    launch_sweep(d.fwd, d.prec, d.fp16, d.rp.get(), d.y.get(), st, err, d.f_sched, s);
-    launch_sweep(d.bck, d.prec, d.fp16, d.y.get(), d.z.get(), st, err, d.b_sched, s);
+    enqueue_pair(d.rp.as<double>(), st, 0, s);
     if (center) launch_sum_out(d.prec, n, d.z.get(), st, part, s);
     launch_apply_gather(d.prec, n, d.perm.as<unsigned>(), d.z.get(), d_z, st, center, s);
 }
@@ -2013,8 +2100,7 @@ void gpu_solver::solve_LLt_device(const double* d_x, double* d_y, hipStream_t s)
     launch_permute(m, Q, d_x, d.rp.as<double>(), true, s);
     launch_fill_pending(d.prec, d.y.get(), m, s);
     launch_fill_pending(d.prec, d.z.get(), m, s);
-    launch_sweep(d.fwd, d.prec, d.fp16, d.rp.get(), d.y.get(), nullptr, d.err.as<int>(), d.f_sched, s);
-    launch_sweep(d.bck, d.prec, d.fp16, d.y.get(), d.z.get(), nullptr, d.err.as<int>(), d.b_sched, s);
+    enqueue_pair(d.rp.as<double>(), nullptr, 0, s);
     launch_permute_out(d.prec, m, Q, d.z.get(), d_y, s);
 }
 
@@ -2048,12 +2134,20 @@ group_member_view gpu_solver::group_view() const {
     v.lumped_offdiag = F_.lumped_offdiag;
     const int m = static_cast<int>(T_.m);
     const std::size_t vsz = d.prec == vec_prec::fp64 ? sizeof(double) : sizeof(float);
+    v.trail.t = d.trail;
+    v.trail.fwd = d.fwd;
+    v.trail.r = d.r.as<double>();
+    v.trail.y = d.y.get();
+    v.trail.c = d.tr_c.as<double>();
+    v.trail.z = d.z.get();
     for (int dir = 0; dir < 2; ++dir) {
         const sweep_sched& sc = dir ? d.b_sched : d.f_sched;
         const sweep_desc& desc = dir ? d.bck : d.fwd;
         if (desc.nb == 0) continue;
         if (sc.kind != 2) throw std::invalid_argument("gpu_solver::group: a group member's sweeps must be the hybrid schedule");
-        for (int k = 0; k < sc.nseg; ++k) {
+        const bool block = d.trail.n > 0;
+        const int k0 = block && dir ? sc.cut_seg : 0, k1 = block && !dir ? sc.cut_seg : sc.nseg;
+        for (int k = k0; k < k1; ++k) {
             if (sc.seg_tail[k]) {
                 group_unit u;
                 u.kind = kGroupTail;

@@ -88,6 +88,13 @@ struct solver_stats {
     int spmv_format = 0;                    // single SpMV: 0 CSR lanes, 1 sliced ELL
     std::uint64_t spmv_sell_slots = 0;      // padded entries of the sliced-ELL form (0: none)
     std::int64_t split_couplings[2] = {0, 0};   // tail runs whose coupling is split, per direction
+    // The trailing block of an application (0 rows: none) and the bytes of its
+    // inverse. The counts above describe whole sweeps (sweep_device); an
+    // application runs the levels outside the block: solve_*.
+    std::int64_t trail_rows = 0;
+    std::uint64_t trail_bytes = 0;
+    std::uint64_t solve_level_bytes[2] = {0, 0}, solve_tail_bytes[2] = {0, 0};
+    std::int64_t solve_level_launches[2] = {0, 0}, solve_tail_runs[2] = {0, 0};
 };
 
 struct block_sched;
@@ -101,7 +108,8 @@ struct group_member_view {
     bool sddm = true;
     vec_prec prec = vec_prec::fp64;
     bool fp16 = false;
-    std::vector<group_unit> steps[2];  // forward, back (st left null)
+    std::vector<group_unit> steps[2];  // forward, back, outside the trailing block (st left null)
+    group_trail trail;                 // t.n == 0: no block (st left null)
     int stagnation_window = 50;
     int center_k = 10;
     std::int64_t lumped_offdiag = 0;
@@ -253,6 +261,13 @@ private:
     // y = A x with the solver's single-vector SpMV (sliced ELL or CSR lanes).
     void spmv(const double* x, double* y, pcg_state* st, bool want_dot, hipStream_t s, const launch_hook& hook) const;
     void enqueue_precondition(bool first, int step, hipStream_t s) const;
+    // Forms the trailing block of the rows from `first` on; false (and no
+    // block) when its inverse leaves the vectors' range.
+    bool build_trail(std::uint32_t first);
+    // z = (L L^T)^-1 r in storage order: the forward levels, the trailing
+    // block, the back levels; one vector, and kp columns of block `which`.
+    void enqueue_pair(const double* r, const pcg_state* st, int step, hipStream_t s) const;
+    void enqueue_pair_k(int kp, const pcg_state* st, const batch_state* bs, hipStream_t s, int which = 0) const;
     std::vector<solve_result> solve_block(int k, const double* d_B, double* d_X, double tol, int max_iter,
                                           hipStream_t s) const;
     int prepare_block(int k, int which = 0) const;

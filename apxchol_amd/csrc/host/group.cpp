@@ -72,6 +72,10 @@ struct solver_group::impl {
     };
     std::vector<step> steps[2];
     devmem units[2];
+    // The members' trailing blocks.
+    devmem trails;
+    int tr_count = 0, tr_couple_s = 0, tr_couple_blocks = 0, tr_apply_s = 0, tr_apply_blocks = 0;
+    std::size_t tr_lds = 0;
     hipStream_t cap = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
@@ -99,6 +103,8 @@ struct solver_group::impl {
     void precondition(bool first, hipStream_t s) const {
         if (first) launch_group_fill_outputs(prec, M(), S(vec_s), count, vec_blocks, s);
         sweep(0, s);
+        launch_group_trail(prec, fp16, trails.as<group_trail>(), S(tr_couple_s), S(tr_apply_s), tr_count,
+                           tr_couple_blocks, tr_apply_blocks, tr_lds, s);
         sweep(1, s);
         launch_group_dot_center(prec, M(), S(vec_s), count, vec_blocks, s);
         launch_group_finish(group_fin_op(first ? "dot_first" : "dot"), M(), S(vec_s), count, s);
@@ -191,6 +197,24 @@ solver_group::solver_group(std::vector<std::shared_ptr<const gpu_solver>> member
             P.steps[dir].push_back(t);
         }
         P.units[dir].upload(units);
+    }
+    {
+        std::vector<group_trail> tr;
+        std::vector<int> g_couple, g_apply;
+        for (int i = 0; i < P.count; ++i) {
+            group_trail u = P.views[i].trail;
+            if (u.t.n == 0) continue;
+            u.st = st + i;
+            g_couple.push_back(trail_couple_blocks(u.t));
+            g_apply.push_back(trail_blocks(u.t, P.prec));
+            P.tr_lds = std::max(P.tr_lds, trail_lds(u.t, P.prec));
+            tr.push_back(u);
+        }
+        P.tr_count = static_cast<int>(tr.size());
+        P.tr_couple_s = add(g_couple, P.tr_couple_blocks);
+        P.tr_apply_s = add(g_apply, P.tr_apply_blocks);
+        P.trails.upload(tr);
+        launches += 2 * (P.tr_count > 0);
     }
     P.starts.upload(all);
     launches_per_iteration_ = launches;

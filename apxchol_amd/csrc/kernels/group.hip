@@ -140,4 +140,27 @@ __global__ __launch_bounds__(kTailBlock) void group_sweep_tail(const group_unit*
                         static_cast<TO*>(u.out), static_cast<const tail_val<TO>*>(u.tv), u.st, 1, nullptr);
 }
 
+// The members' trailing blocks (kernels/trail.hip): the coupling launch, then
+// the product.
+template <class TO, bool F16>
+__global__ __launch_bounds__(kCoupleThreads) void group_trail_couple(const group_trail* __restrict__ units,
+                                                                     const int* __restrict__ starts, int count) {
+    const int b = static_cast<int>(blockIdx.x);
+    const int i = group_unit_of(starts, count, b);
+    const group_trail& u = units[i];
+    trail_couple_body<TO, F16>(b - starts[i], 0, u.t, u.fwd, u.r, static_cast<const TO*>(u.y), u.c,
+                               u.st, 1, nullptr);
+}
+
+template <class TO>
+__global__ __launch_bounds__(kTrailThreads) void group_trail_apply(const group_trail* __restrict__ units,
+                                                                   const int* __restrict__ starts, int count) {
+    extern __shared__ unsigned char group_trail_lds[];
+    const int b = static_cast<int>(blockIdx.x);
+    const int i = group_unit_of(starts, count, b);
+    const group_trail& u = units[i];
+    trail_apply_body<TO>(b - starts[i], group_trail_lds, u.t, u.c, static_cast<TO*>(u.z),
+                         u.st);
+}
+
 }  // namespace apxchol_amd

@@ -13,6 +13,7 @@
 #include "pcg.hip"
 #include "sweep.hip"
 #include "block.hip"
+#include "trail.hip"
 #include "pieces.hip"
 #include "group.hip"
 
@@ -67,9 +68,16 @@ inline constexpr int kLevelMaxBlocks = kLevelLaunchMaxBlocks;
 
 template <class TI, class TO, bool F16>
 void sweep_t(const sweep_desc& d, const void* rhs, void* out, const pcg_state* st, int* err, const sweep_sched& sc,
-             hipStream_t s, const launch_hook& hook) {
+             hipStream_t s, const launch_hook& hook, sweep_part rows) {
     const TI* in = static_cast<const TI*>(rhs);
     TO* o = static_cast<TO*>(out);
+    // The trailing block is the end of the forward sweep and the start of the
+    // back sweep.
+    const bool outside = rows == sweep_part::outside_block;
+    const auto range = [&](int cut, int end, int& lo, int& hi) {
+        lo = outside && d.backward ? cut : 0;
+        hi = outside && !d.backward ? cut : end;
+    };
     auto level_launch = [&](int l) {
         const int b0 = sc.level_first[l], b1 = sc.level_first[l + 1];
         if (b1 <= b0) return;
@@ -104,11 +112,16 @@ void sweep_t(const sweep_desc& d, const void* rhs, void* out, const pcg_state* s
         launch_timed(hook, 0, sweep_levels<TI, TO, F16>, dim3(g), dim3(kBlock), 0, s, d, b0, b1, in, o, st, err);
     };
     if (sc.kind == 0) {
-        launch_timed(hook, 3, sweep_dataflow<TI, TO, F16>, dim3(sc.grid), dim3(kBlock), 0, s, d, in, o, st,
+        sweep_desc part = d;
+        range(sc.cut_batch, d.nb, part.b_first, part.nb);
+        if (part.b_first >= part.nb) return;
+        launch_timed(hook, 3, sweep_dataflow<TI, TO, F16>, dim3(sc.grid), dim3(kBlock), 0, s, part, in, o, st,
                      sc.grid * kWavesPerBlock, err);
         check_launch("sweep_dataflow");
     } else if (sc.kind == 1) {
-        for (int l = 0; l < sc.nlevels; ++l) level_launch(l);
+        int l0, l1;
+        range(sc.cut_level, sc.nlevels, l0, l1);
+        for (int l = l0; l < l1; ++l) level_launch(l);
         check_launch("sweep_levels");
     } else {
         static const bool attr = [] {
@@ -128,13 +141,15 @@ void sweep_t(const sweep_desc& d, const void* rhs, void* out, const pcg_state* s
             tv = static_cast<tail_val<TO>*>(sc.tail_val) + static_cast<size_t>(base) * kWave;
         };
         const bool can_split = sc.seg_split && sc.side && sc.ev_fork && sc.ev_join;
-        const auto split_at = [&](int k) { return can_split && k < sc.nseg && sc.seg_tail[k] ? sc.seg_split[k] : -1; };
+        int k0, k1;
+        range(sc.cut_seg, sc.nseg, k0, k1);
+        const auto split_at = [&](int k) { return can_split && k < k1 && sc.seg_tail[k] ? sc.seg_split[k] : -1; };
         // One wave per workgroup (a batch each), as the lane levels.
         const auto couple = [&](hipStream_t on, int bf, int bl, int plo, int phi, int cont, tail_val<TO>* tv) {
             launch_timed(hook, 2, sweep_couple<TI, TO, F16, kWave>, dim3(bl - bf), dim3(kWave), 0, on, d, bf, bl, plo,
                          phi, cont, in, static_cast<const TO*>(o), tv, st, 1, static_cast<const batch_state*>(nullptr));
         };
-        for (int k = 0; k < sc.nseg; ++k) {
+        for (int k = k0; k < k1; ++k) {
             if (!sc.seg_tail[k]) {
                 for (int l = sc.seg_l0[k]; l < sc.seg_l1[k]; ++l) level_launch(l);
                 continue;
@@ -198,17 +213,17 @@ bool sweep_tail_fits(vec_prec p, int rows, int batches, int levels) {
 }
 
 void launch_sweep(const sweep_desc& d, vec_prec p, bool fp16, const void* rhs, void* out, const pcg_state* st,
-                  int* err, const sweep_sched& sc, hipStream_t s, const launch_hook& hook) {
+                  int* err, const sweep_sched& sc, hipStream_t s, const launch_hook& hook, sweep_part rows) {
     if (d.nb == 0) return;
     if (p == vec_prec::fp64) {
-        if (fp16) sweep_t<double, double, true>(d, rhs, out, st, err, sc, s, hook);
-        else sweep_t<double, double, false>(d, rhs, out, st, err, sc, s, hook);
+        if (fp16) sweep_t<double, double, true>(d, rhs, out, st, err, sc, s, hook, rows);
+        else sweep_t<double, double, false>(d, rhs, out, st, err, sc, s, hook, rows);
     } else if (!d.backward) {
-        if (fp16) sweep_t<double, float, true>(d, rhs, out, st, err, sc, s, hook);
-        else sweep_t<double, float, false>(d, rhs, out, st, err, sc, s, hook);
+        if (fp16) sweep_t<double, float, true>(d, rhs, out, st, err, sc, s, hook, rows);
+        else sweep_t<double, float, false>(d, rhs, out, st, err, sc, s, hook, rows);
     } else {
-        if (fp16) sweep_t<float, float, true>(d, rhs, out, st, err, sc, s, hook);
-        else sweep_t<float, float, false>(d, rhs, out, st, err, sc, s, hook);
+        if (fp16) sweep_t<float, float, true>(d, rhs, out, st, err, sc, s, hook, rows);
+        else sweep_t<float, float, false>(d, rhs, out, st, err, sc, s, hook, rows);
     }
 }
 
@@ -373,13 +388,128 @@ void launch_fill_pending(vec_prec p, void* a, int n, hipStream_t s) {
     check_launch("fill_pending");
 }
 
+// ---- the trailing block -------------------------------------------------------
+
+int trail_rows_per_block(vec_prec p) { return kTrailLine / static_cast<int>(p == vec_prec::fp64 ? sizeof(double) : sizeof(float)); }
+
+int trail_chunks(vec_prec p) { return kTrailThreads / trail_rows_per_block(p); }
+
+int trail_blocks(const trail_desc& t, vec_prec p) {
+    return (t.n + trail_rows_per_block(p) - 1) / trail_rows_per_block(p);
+}
+
+std::size_t trail_lds(const trail_desc& t, vec_prec p) {
+    return std::max<std::size_t>(static_cast<std::size_t>(trail_chunks(p)) * t.chunk, kTrailThreads) * sizeof(double);
+}
+
+int trail_couple_blocks(const trail_desc& t) {
+    constexpr int waves = kCoupleThreads / kWave;
+    return (t.npack + waves - 1) / waves + t.nlong;
+}
+
+namespace {
+// The product's LDS holds c: up to kTrailMaxRows values, rounded up to whole chunks.
+inline constexpr int kTrailLdsMax = 96 * 1024;
+
+void check_trail(const trail_desc& t, vec_prec p) {
+    if (t.n < 1 || t.n > kTrailMaxRows || t.ld % kWave != 0 || t.ld < t.n || t.chunk < 4 || t.chunk % 4 != 0 ||
+        trail_chunks(p) * t.chunk < t.n || trail_lds(t, p) > static_cast<std::size_t>(kTrailLdsMax) || !t.s)
+        throw std::runtime_error("apxchol_amd: inconsistent trailing block");
+}
+
+template <class K>
+void trail_lds_attr(K kernel) {
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              kTrailLdsMax);
+}
+
+template <class TO>
+void trail_t(const trail_desc& t, const sweep_desc& fwd, bool fp16, const double* r, const TO* y, double* c, TO* z,
+             const pcg_state* st, hipStream_t s, const launch_hook& hook) {
+    const vec_prec p = sizeof(TO) == sizeof(double) ? vec_prec::fp64 : vec_prec::fp32;
+    check_trail(t, p);
+    const dim3 g(static_cast<unsigned>(trail_couple_blocks(t)));
+    const batch_state* none = nullptr;
+    auto couple = [&](auto kernel) { launch_timed(hook, 2, kernel, g, dim3(kCoupleThreads), 0, s, t, fwd, r, y, c, st, 1, none); };
+    if (fp16) couple(trail_couple<TO, true>);
+    else couple(trail_couple<TO, false>);
+    static const bool attr = [] { trail_lds_attr(&trail_apply<TO>); return true; }();
+    (void)attr;
+    launch_timed(hook, 1, trail_apply<TO>, dim3(static_cast<unsigned>(trail_blocks(t, p))), dim3(kTrailThreads),
+                 static_cast<unsigned>(trail_lds(t, p)), s, t, static_cast<const double*>(c), z, st);
+    check_launch("trail");
+}
+
+template <class TO>
+void trail_k_t(const trail_desc& t, const sweep_desc& fwd, bool fp16, int kp, const double* r, const TO* y, double* c,
+               TO* z, const pcg_state* st, const batch_state* bs, hipStream_t s) {
+    check_trail(t, sizeof(TO) == sizeof(double) ? vec_prec::fp64 : vec_prec::fp32);
+    const dim3 g(static_cast<unsigned>(trail_couple_blocks(t)), static_cast<unsigned>(kp));
+    if (fp16) trail_couple<TO, true><<<g, kCoupleThreads, 0, s>>>(t, fwd, r, y, c, st, kp, bs);
+    else trail_couple<TO, false><<<g, kCoupleThreads, 0, s>>>(t, fwd, r, y, c, st, kp, bs);
+    constexpr int kCols = 8;   // columns per workgroup: 16 waves' sums in 64 KB of LDS
+    const unsigned tiles = static_cast<unsigned>((t.n + kWave - 1) / kWave);
+    const double* cc = c;
+    auto apply = [&](auto kernel, int ct) { kernel<<<dim3(tiles, static_cast<unsigned>(kp / ct)), kTrailThreads, 0, s>>>(t, cc, z, kp, bs); };
+    const int ct = std::min(kp, kCols);
+    if (ct == 1) apply(trail_apply_k<TO, 1>, 1);
+    else if (ct == 2) apply(trail_apply_k<TO, 2>, 2);
+    else if (ct == 4) apply(trail_apply_k<TO, 4>, 4);
+    else apply(trail_apply_k<TO, kCols>, kCols);
+    check_launch("trail_k");
+}
+}  // namespace
+
+void launch_trail(const trail_desc& t, const sweep_desc& fwd, vec_prec p, bool fp16, const double* r, const void* y,
+                  double* c, void* z, const pcg_state* st, hipStream_t s, const launch_hook& hook) {
+    if (p == vec_prec::fp64)
+        trail_t<double>(t, fwd, fp16, r, static_cast<const double*>(y), c, static_cast<double*>(z), st, s, hook);
+    else
+        trail_t<float>(t, fwd, fp16, r, static_cast<const float*>(y), c, static_cast<float*>(z), st, s, hook);
+}
+
+void launch_trail_setup(const sweep_desc& fwd, const float* inv_scale, vec_prec p, bool fp16, int first, int n, int np,
+                        double* a, double* x, void* s, std::size_t s_values, int ld, int* bad, hipStream_t st) {
+    if (n < 1 || np % kWave != 0 || np < n || ld < np || first < 0 || first + n != fwd.m)
+        throw std::runtime_error("apxchol_amd: inconsistent trailing block setup");
+    const std::size_t cells = static_cast<std::size_t>(np) * np;
+    const auto zero = [&](double* q, std::size_t count) { trail_zero<<<2048, kBlock, 0, st>>>(q, count); };
+    zero(a, cells);
+    zero(x, cells);
+    // The padding of S past np (values of either width: whole doubles, the
+    // buffer is a multiple of 8 bytes).
+    zero(static_cast<double*>(s), s_values * (p == vec_prec::fp64 ? 8 : 4) / 8);
+    zero(reinterpret_cast<double*>(bad), 1);
+    const int gs = (np + kWavesPerBlock - 1) / kWavesPerBlock;
+    if (fp16) trail_scatter<true><<<gs, kBlock, 0, st>>>(fwd, first, n, np, a);
+    else trail_scatter<false><<<gs, kBlock, 0, st>>>(fwd, first, n, np, a);
+    trail_invert_diag<<<np / kWave, kWave, 0, st>>>(np, a, x);
+    for (int w = kWave; w < np; w *= 2) {
+        const unsigned pairs = static_cast<unsigned>((np - w + 2 * w - 1) / (2 * w));
+        const dim3 g(static_cast<unsigned>(w / kWave), static_cast<unsigned>(w / kWave), pairs);
+        trail_invert_step<<<g, kBlock, 0, st>>>(np, w, 0, a, x);
+        trail_invert_step<<<g, kBlock, 0, st>>>(np, w, 1, a, x);
+    }
+    const dim3 g(static_cast<unsigned>(np / kWave), static_cast<unsigned>(np / kWave));
+    const float* w = inv_scale ? inv_scale + first : nullptr;
+    if (p == vec_prec::fp64) trail_form<double><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<double*>(s), ld, bad);
+    else trail_form<float><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<float*>(s), ld, bad);
+    check_launch("trail_setup");
+}
+
 // ---- blocked solves ---------------------------------------------------------
 
 namespace {
 
 template <class TI, class TO, bool F16>
 void sweep_k_t(const sweep_desc& d, const block_sched& b, const void* rhs, void* out, const pcg_state* st,
-               const batch_state* bs, hipStream_t s) {
+               const batch_state* bs, hipStream_t s, sweep_part rows) {
+    const bool outside = rows == sweep_part::outside_block;
+    const auto range = [&](int cut, int end, int& lo, int& hi) {
+        lo = outside && d.backward ? cut : 0;
+        hi = outside && !d.backward ? cut : end;
+    };
+    int first, last;
     auto level_launch = [&](int l) {
         const int w0 = b.level_first[l], w1 = b.level_first[l + 1];
         if (w1 <= w0) return;
@@ -420,7 +550,8 @@ void sweep_k_t(const sweep_desc& d, const block_sched& b, const void* rhs, void*
             return true;
         }();
         (void)attr;
-        for (int k = 0; k < sc.nseg; ++k) {
+        range(sc.cut_seg, sc.nseg, first, last);
+        for (int k = first; k < last; ++k) {
             if (!sc.seg_tail[k]) {
                 for (int l = sc.seg_l0[k]; l < sc.seg_l1[k]; ++l) level_launch(l);
                 continue;
@@ -442,7 +573,8 @@ void sweep_k_t(const sweep_desc& d, const block_sched& b, const void* rhs, void*
                                                          st, b.kp, bs);
         }
     } else if (b.nseg == 0) {
-        for (int l = 0; l < b.nlevels; ++l) level_launch(l);
+        range(b.cut_level, b.nlevels, first, last);
+        for (int l = first; l < last; ++l) level_launch(l);
     } else {
         static const bool attr = [] {
             (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&sweep_block_tail<TI, TO, F16>),
@@ -450,7 +582,8 @@ void sweep_k_t(const sweep_desc& d, const block_sched& b, const void* rhs, void*
             return true;
         }();
         (void)attr;
-        for (int k = 0; k < b.nseg; ++k) {
+        range(b.cut_seg, b.nseg, first, last);
+        for (int k = first; k < last; ++k) {
             const int l0 = b.seg_l0[k], l1 = b.seg_l1[k];
             if (!b.seg_tail[k]) {
                 for (int l = l0; l < l1; ++l) level_launch(l);
@@ -487,18 +620,27 @@ int sweep_block_tail_max_rows(vec_prec p, int kp) {
 }
 
 void launch_sweep_k(const sweep_desc& d, vec_prec p, bool fp16, const block_sched& b, const void* rhs, void* out,
-                    const pcg_state* st, const batch_state* bs, hipStream_t s) {
+                    const pcg_state* st, const batch_state* bs, hipStream_t s, sweep_part rows) {
     check_kp(b.kp);
     if (p == vec_prec::fp64) {
-        if (fp16) sweep_k_t<double, double, true>(d, b, rhs, out, st, bs, s);
-        else sweep_k_t<double, double, false>(d, b, rhs, out, st, bs, s);
+        if (fp16) sweep_k_t<double, double, true>(d, b, rhs, out, st, bs, s, rows);
+        else sweep_k_t<double, double, false>(d, b, rhs, out, st, bs, s, rows);
     } else if (!d.backward) {
-        if (fp16) sweep_k_t<double, float, true>(d, b, rhs, out, st, bs, s);
-        else sweep_k_t<double, float, false>(d, b, rhs, out, st, bs, s);
+        if (fp16) sweep_k_t<double, float, true>(d, b, rhs, out, st, bs, s, rows);
+        else sweep_k_t<double, float, false>(d, b, rhs, out, st, bs, s, rows);
     } else {
-        if (fp16) sweep_k_t<float, float, true>(d, b, rhs, out, st, bs, s);
-        else sweep_k_t<float, float, false>(d, b, rhs, out, st, bs, s);
+        if (fp16) sweep_k_t<float, float, true>(d, b, rhs, out, st, bs, s, rows);
+        else sweep_k_t<float, float, false>(d, b, rhs, out, st, bs, s, rows);
     }
+}
+
+void launch_trail_k(const trail_desc& t, const sweep_desc& fwd, vec_prec p, bool fp16, int kp, const double* r,
+                    const void* y, double* c, void* z, const pcg_state* st, const batch_state* bs, hipStream_t s) {
+    check_kp(kp);
+    if (p == vec_prec::fp64)
+        trail_k_t<double>(t, fwd, fp16, kp, r, static_cast<const double*>(y), c, static_cast<double*>(z), st, bs, s);
+    else
+        trail_k_t<float>(t, fwd, fp16, kp, r, static_cast<const float*>(y), c, static_cast<float*>(z), st, bs, s);
 }
 
 void launch_spmm_k(int n, int kp, int lanes, const unsigned* ptr, const int* idx, const void* val, bool val32,
@@ -907,6 +1049,28 @@ void launch_group_sweep_tail(vec_prec p, const group_unit* units, int count, std
         group_sweep_tail<float><<<count, kTailBlock, static_cast<unsigned>(lds), s>>>(units);
     }
     check_launch("group_sweep_tail");
+}
+
+void launch_group_trail(vec_prec p, bool fp16, const group_trail* units, const int* couple_starts,
+                        const int* apply_starts, int count, int couple_blocks, int apply_blocks, std::size_t lds,
+                        hipStream_t s) {
+    if (count <= 0) return;
+    if (lds > static_cast<std::size_t>(kTrailLdsMax)) throw std::runtime_error("apxchol_amd: group trailing block exceeds LDS");
+    auto couple = [&](auto kernel) { kernel<<<couple_blocks, kCoupleThreads, 0, s>>>(units, couple_starts, count); };
+    if (p == vec_prec::fp64) {
+        if (fp16) couple(group_trail_couple<double, true>);
+        else couple(group_trail_couple<double, false>);
+        static const bool attr = [] { trail_lds_attr(&group_trail_apply<double>); return true; }();
+        (void)attr;
+        group_trail_apply<double><<<apply_blocks, kTrailThreads, static_cast<unsigned>(lds), s>>>(units, apply_starts, count);
+    } else {
+        if (fp16) couple(group_trail_couple<float, true>);
+        else couple(group_trail_couple<float, false>);
+        static const bool attr = [] { trail_lds_attr(&group_trail_apply<float>); return true; }();
+        (void)attr;
+        group_trail_apply<float><<<apply_blocks, kTrailThreads, static_cast<unsigned>(lds), s>>>(units, apply_starts, count);
+    }
+    check_launch("group_trail");
 }
 
 }  // namespace apxchol_amd

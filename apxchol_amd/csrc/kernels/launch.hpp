@@ -56,7 +56,13 @@ struct sweep_sched {
     long long lane_batches = 0;
     int lane_bpw2 = 0;                     // lane levels of >= this many batches: 2 per wave (0: never)
     int lane_bpw4 = 0;                     // ... >= this many: 4 per wave (0: never)
+    // The boundary of the trailing block in this direction: its first level,
+    // segment and batch (back sweep: the first ones after it).
+    int cut_level = 0, cut_seg = 0, cut_batch = 0;
 };
+// The rows a sweep launch covers: all, or those outside the trailing block
+// (the back sweep then expects the block's outputs in place).
+enum class sweep_part { whole, outside_block };
 
 // Kernel timing: for kernel `kind` (0 sweep_levels, 1 sweep_tail,
 // 2 sweep_couple, 3 sweep_dataflow, 4 spmv_pAp) the hook may hand out a
@@ -72,7 +78,29 @@ struct launch_hook {
 // as `p`); out: fp64 or fp32 as `p` (every slot pending on entry for the
 // dataflow schedule).
 void launch_sweep(const sweep_desc& d, vec_prec p, bool fp16, const void* rhs, void* out, const pcg_state* st,
-                  int* err, const sweep_sched& sc, hipStream_t s, const launch_hook& hook = {});
+                  int* err, const sweep_sched& sc, hipStream_t s, const launch_hook& hook = {},
+                  sweep_part rows = sweep_part::whole);
+
+// The trailing block (kernels/trail.hip): its outputs z from r and the forward
+// outputs y of the rows before it, through c (n values); kinds 2 and 1 of the
+// hook. With kp > 1 columns (row-major blocks, c of n * kp values) st holds
+// one state per column and bs stops the launches.
+void launch_trail(const trail_desc& t, const sweep_desc& fwd, vec_prec p, bool fp16, const double* r, const void* y,
+                  double* c, void* z, const pcg_state* st, hipStream_t s, const launch_hook& hook = {});
+void launch_trail_k(const trail_desc& t, const sweep_desc& fwd, vec_prec p, bool fp16, int kp, const double* r,
+                    const void* y, double* c, void* z, const pcg_state* st, const batch_state* bs, hipStream_t s);
+// Rows one workgroup of the product owns, the padded rows of S, its workgroups
+// and its LDS bytes; the workgroups of the coupling launch.
+int trail_rows_per_block(vec_prec p);
+int trail_chunks(vec_prec p);
+int trail_blocks(const trail_desc& t, vec_prec p);
+std::size_t trail_lds(const trail_desc& t, vec_prec p);
+int trail_couple_blocks(const trail_desc& t);
+// Forms S of the rows [first, first + n) of the factor: a, x are scratch of
+// np * np doubles (np: n rounded up to 64), s the zero-filled output; *bad
+// becomes non-zero when an entry is not finite.
+void launch_trail_setup(const sweep_desc& fwd, const float* inv_scale, vec_prec p, bool fp16, int first, int n, int np,
+                        double* a, double* x, void* s, std::size_t s_values, int ld, int* bad, hipStream_t st);
 
 // z past the sweep rows = 0; with y given, y and z pending (dataflow only).
 void launch_fill_outputs(vec_prec p, int n, int m, void* y, void* z, const pcg_state* st, hipStream_t s);
@@ -135,6 +163,7 @@ struct block_sched {
     const int* seg_l1 = nullptr;
     const int* seg_tail = nullptr;
     int nseg = 0;
+    int cut_level = 0, cut_seg = 0;         // the trailing block's boundary, as in sweep_sched
     // When set: the single-vector schedule whose levels this sweep follows,
     // its tail runs walked column by column (one tail workgroup per column)
     // with the coupling values in col_tail_val (kp * 64 tail_val per run batch).
@@ -144,7 +173,8 @@ struct block_sched {
 };
 // One blocked sweep as one launch per level.
 void launch_sweep_k(const sweep_desc& d, vec_prec p, bool fp16, const block_sched& bsc, const void* rhs, void* out,
-                    const pcg_state* st, const batch_state* bs, hipStream_t s);
+                    const pcg_state* st, const batch_state* bs, hipStream_t s,
+                    sweep_part rows = sweep_part::whole);
 // Rows a blocked tail run of block width kp may hold (LDS).
 int sweep_block_tail_max_rows(vec_prec p, int kp);
 void launch_spmm_k(int n, int kp, int lanes, const unsigned* ptr, const int* idx, const void* val, bool val32,
@@ -200,6 +230,16 @@ struct group_member {
     const void* oval = nullptr;
 };
 inline constexpr int kGroupLane = 0, kGroupLevels = 1, kGroupTail = 2;
+// One member's trailing block in a grouped launch.
+struct group_trail {
+    trail_desc t;
+    sweep_desc fwd;
+    const double* r = nullptr;
+    const void* y = nullptr;
+    double* c = nullptr;
+    void* z = nullptr;
+    const pcg_state* st = nullptr;
+};
 // Workgroups of one level launch from the batch tables: one wave per batch, at most this many;
 // waves per workgroup of the level launches.
 inline constexpr int kLevelLaunchMaxBlocks = 16384;
@@ -242,6 +282,10 @@ void launch_group_sweep_level(vec_prec p, bool fp16, bool backward, const group_
 void launch_group_sweep_couple(vec_prec p, bool fp16, bool backward, const group_unit* units, const int* starts,
                                int count, int blocks, hipStream_t s);
 void launch_group_sweep_tail(vec_prec p, const group_unit* units, int count, std::size_t lds, hipStream_t s);
+// The members' trailing blocks: one coupling launch and one product launch.
+void launch_group_trail(vec_prec p, bool fp16, const group_trail* units, const int* couple_starts,
+                        const int* apply_starts, int count, int couple_blocks, int apply_blocks, std::size_t lds,
+                        hipStream_t s);
 // The reduction-stage op codes of pcg_finish (kFinPAp ...), for the group host.
 int group_fin_op(const char* name);
 

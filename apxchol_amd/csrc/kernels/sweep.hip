@@ -331,7 +331,7 @@ __global__ __launch_bounds__(kBlock) void sweep_dataflow(sweep_desc d, const TI*
     for (;;) {
         int b0 = 0;
         if (lane == 0) b0 = atomicAdd(&d.ctrl[0], d.chunk);
-        b0 = __shfl(b0, 0, kWave);
+        b0 = __shfl(b0, 0, kWave) + d.b_first;
         if (b0 >= d.nb) break;
         const int b1 = min(b0 + d.chunk, d.nb);
         for (int b = b0; b < b1; ++b) {

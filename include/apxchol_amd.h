@@ -150,6 +150,19 @@ apx_status apx_solver_create_with_factor(int64_t n, const int64_t* colptr, const
 void apx_solver_destroy(apx_solver_t s);
 apx_status apx_solver_info_get(apx_solver_t s, apx_solver_info* info);
 
+/* What one preconditioner application runs. The last `rows` rows of the factor
+ * (0: none) are applied through their explicit inverse, `bytes` of it, by one
+ * coupling launch and one matrix-vector product; the levels before them as
+ * apx_solver_info describes whole sweeps: per direction [0 forward, 1 back]
+ * the bytes and counts of the level launches and tail runs outside the block. */
+typedef struct {
+    int64_t rows;
+    uint64_t bytes;
+    uint64_t level_bytes[2], tail_bytes[2];
+    int64_t level_launches[2], tail_runs[2];
+} apx_block_info;
+apx_status apx_solver_block_get(apx_solver_t s, apx_block_info* info);
+
 /* cpu_solver::solve(b, x, tol, max_iter, x0) (solve.h:83-100, src/solve.cpp:478-654),
  * on device vectors of n doubles. tol < 0 / max_iter < 0 use the options;
  * d_x0 may be NULL. The PCG runs on the GPU (cuda_pcg::solve, pcg_cuda.h:157-261). */
