@@ -807,12 +807,16 @@ void gpu_solver::setup(const csc_view& L) {
     // XCD's share, see spmv_sell -- gathers from a band of vertices and its
     // neighbours; unsorted when 64-row slices pad to <= 1.2 x the entries,
     // else sorted by length inside 4096-row windows (rows longer than
-    // max(64, 8 mean) walked by a wave) when that pads to <= 1.5 x; otherwise
+    // max(32, mean) walked by a wave) when that pads to <= 1.5 x; otherwise
     // CSR lanes only. APXCHOL_AMD_SPMV=csr / sell forces the choice;
     // APXCHOL_AMD_SELL_ORDER=storage slices in storage order instead.
     {
         const std::int64_t nnz = op.ptr.back();
-        const std::int64_t long_len = std::max<std::int64_t>(64, 8 * static_cast<std::int64_t>(std::ceil(avg)));
+        // A lane walks its row of a slice alone, a wave the rows past the mean:
+        // the longest lane chain is the launch's critical path (SpMV calls at
+        // max(64, 8 mean) / max(64, 2 mean) / max(32, mean): R-MAT s14 28.9 /
+        // 16.9 / 14.1 us, s18 122 / 79 / 80).
+        const std::int64_t long_len = std::max<std::int64_t>(32, static_cast<std::int64_t>(std::ceil(avg)));
         const char* fe = std::getenv("APXCHOL_AMD_SPMV");
         const std::string force = fe ? fe : "";
         const char* oe = std::getenv("APXCHOL_AMD_SELL_ORDER");

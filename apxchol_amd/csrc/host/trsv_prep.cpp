@@ -362,6 +362,8 @@ sell_layout build_sell(const permuted_operator& op, std::int64_t long_len, std::
             std::stable_sort(order.begin() + static_cast<std::ptrdiff_t>(first), order.end(),
                              [&](std::int32_t a, std::int32_t b) { return len(a) > len(b); });
     }
+    std::stable_sort(s.longrows.begin(), s.longrows.end(),
+                     [&](std::int32_t a, std::int32_t b) { return len(a) > len(b); });
     const std::int64_t nrows = static_cast<std::int64_t>(order.size());
     const std::int64_t nslices = (nrows + 63) / 64;
     s.soff.assign(static_cast<std::size_t>(nslices) + 1, 0);

@@ -79,7 +79,7 @@ struct permuted_operator {
 permuted_operator build_permuted_operator(const csc_view& A, const std::vector<node_t>& perm);
 
 // Sliced-ELL form of the operator (device.hpp's sell_desc): rows with more
-// than long_len entries are listed in longrows; the others are packed 64 to a
+// than long_len entries are listed in longrows, longest first; the others are packed 64 to a
 // slice in the order `rows` gives (a permutation of the n rows; with sigma > 1
 // stably sorted by decreasing length inside windows of sigma of them) and a
 // row map records it.

@@ -465,10 +465,8 @@ __global__ __launch_bounds__(kBlock) void spmm_sell_k(sell_desc a, int kp, const
             const int col = static_cast<int>(li % kp);
             const unsigned b = a.ptr[row], e = a.ptr[row + 1];
             const VT* __restrict__ cval = static_cast<const VT*>(a.cval);
-            double s = 0.0;
-            for (unsigned p = b + lane; p < e; p += kWave)
-                s = fma(static_cast<double>(cval[p]), x[static_cast<size_t>(a.cidx[p]) * kp + col], s);
-            s = wave_sum(s);
+            const double s = wave_sum(long_row_sum<8, VT>(a.cidx, cval, b, e, lane,
+                                                       [&](int j) { return x[static_cast<size_t>(j) * kp + col]; }));
             // The long rows' share of p.Ap comes from spmm_long_dot_k (its
             // waves sit in column-dependent workgroups).
             if (lane == 0) y[static_cast<size_t>(row) * kp + col] = s;
@@ -573,10 +571,8 @@ __global__ __launch_bounds__(kBlock) void spmm_sell_staged_k(sell_desc a, int kp
         const int col = static_cast<int>(li % kp);
         const unsigned b = a.ptr[row], e = a.ptr[row + 1];
         const VT* __restrict__ cval = static_cast<const VT*>(a.cval);
-        double s = 0.0;
-        for (unsigned p = b + lane; p < e; p += kWave)
-            s = fma(static_cast<double>(cval[p]), x[static_cast<size_t>(a.cidx[p]) * kp + col], s);
-        s = wave_sum(s);
+        const double s = wave_sum(long_row_sum<8, VT>(a.cidx, cval, b, e, lane,
+                                                   [&](int j) { return x[static_cast<size_t>(j) * kp + col]; }));
         if (lane == 0) y[static_cast<size_t>(row) * kp + col] = s;
     }
     if (!want_dot) return;

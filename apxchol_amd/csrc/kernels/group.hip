@@ -47,8 +47,13 @@ __global__ __launch_bounds__(kBlock) void group_spmv(const group_member* __restr
     const group_member& g = mem[i];
     const int vb = b - starts[i], vg = starts[i + 1] - starts[i];
     if (g.use_sell) {
-        if (g.val32) spmv_sell_body<float>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
-        else spmv_sell_body<double>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
+        if (g.sell.nlong > 0) {
+            if (g.val32) spmv_sell_body<float, true>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
+            else spmv_sell_body<double, true>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
+        } else {
+            if (g.val32) spmv_sell_body<float, false>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
+            else spmv_sell_body<double, false>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
+        }
     } else {
         if (g.val32) group_spmv_csr<float>(vb, vg, g);
         else group_spmv_csr<double>(vb, vg, g);

@@ -281,8 +281,13 @@ void launch_spmv_sell(const sell_desc& a, bool val32, const double* x, double* y
         launch_timed(hook, 4, kernel, dim3(static_cast<unsigned>(g)), dim3(kBlock), 0, s, a, x, y, st, part, w);
     };
     if (!a.rowmap) throw std::invalid_argument("apxchol_amd: sliced ELL without a row map");
-    if (val32) go(spmv_sell<float>);
-    else go(spmv_sell<double>);
+    if (a.nlong > 0) {
+        if (val32) go(spmv_sell<float, true>);
+        else go(spmv_sell<double, true>);
+    } else {
+        if (val32) go(spmv_sell<float, false>);
+        else go(spmv_sell<double, false>);
+    }
     check_launch("spmv_sell");
     if (want_dot) finish(kFinPAp, a.n, part, static_cast<int>(g), st, s);
 }

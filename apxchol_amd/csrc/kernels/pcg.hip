@@ -56,13 +56,104 @@ __global__ __launch_bounds__(kBlock) void spmv_pAp(int n, const unsigned* __rest
                          want_dot);
 }
 
+// A long row of the operator walked by one wave: lane l sums entries b + l,
+// b + l + 64, ... in order (fma from 0), U of them per round -- the round's
+// index and value loads, then its gathers, in flight together, so a round and
+// not an entry is a dependent round trip, the next round's indices and values
+// fetched beside the gathers -- and the rest of the row 4 at a time
+// (slots past the row repeat its first entry and are left out of the sum).
+// get(j): the vector's element j.
+template <int U, class VT, class X>
+__device__ __forceinline__ void long_row_round(const int* __restrict__ cidx, const VT* __restrict__ cval, unsigned b,
+                                               unsigned e, unsigned p0, int lane, X get, double& s) {
+    int j[U];
+    VT v[U];
+    double g[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const unsigned p = p0 + static_cast<unsigned>(lane + u * kWave);
+        j[u] = cidx[p < e ? p : b];
+        v[u] = cval[p < e ? p : b];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) g[u] = get(j[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+        if (p0 + static_cast<unsigned>(lane + u * kWave) < e) s = fma(static_cast<double>(v[u]), g[u], s);
+}
+template <int U, class VT, class X>
+__device__ __forceinline__ double long_row_sum(const int* __restrict__ cidx, const VT* __restrict__ cval, unsigned b,
+                                               unsigned e, int lane, X get) {
+    double s = 0.0;
+    unsigned p = b;
+    if (p + (U - 4) * kWave < e) {
+        int j[U];
+        VT v[U];
+        const auto fetch = [&](unsigned p0, int (&jj)[U], VT (&vv)[U]) {
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const unsigned q = p0 + static_cast<unsigned>(lane + u * kWave);
+                jj[u] = cidx[q < e ? q : b];
+                vv[u] = cval[q < e ? q : b];
+            }
+        };
+        fetch(p, j, v);
+        do {
+            const unsigned pn = p + U * kWave;
+            double g[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) g[u] = get(j[u]);
+            int jn[U];
+            VT vn[U];
+            fetch(pn < e ? pn : b, jn, vn);
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                if (p + static_cast<unsigned>(lane + u * kWave) < e) s = fma(static_cast<double>(v[u]), g[u], s);
+#pragma unroll
+            for (int u = 0; u < U; ++u) { j[u] = jn[u]; v[u] = vn[u]; }
+            p = pn;
+        } while (p + (U - 4) * kWave < e);
+    }
+    for (; p < e; p += 4u * kWave) long_row_round<4, VT>(cidx, cval, b, e, p, lane, get, s);
+    return s;
+}
+
+// A lane's row of a slice of w columns: columns in groups of U (the last group
+// predicated), all of a group's loads, then its gathers, in flight together.
+template <int U, class VT>
+__device__ __forceinline__ double slice_sum(const int* __restrict__ sidx, const VT* __restrict__ sval, size_t base,
+                                            int w, const double* __restrict__ x) {
+    double s = 0.0;
+    for (int k = 0; k < w; k += U) {
+        int j[U];
+        double v[U], g[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const bool ok = k + u < w;
+            j[u] = ok ? sidx[base + static_cast<size_t>(k + u) * kWave] : 0;
+            v[u] = ok ? static_cast<double>(sval[base + static_cast<size_t>(k + u) * kWave]) : 0.0;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) g[u] = k + u < w ? x[j[u]] : 0.0;
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+            if (k + u < w) s = fma(v[u], g[u], s);
+    }
+    return s;
+}
+
 // y = A x over the sliced-ELL form (sell_desc): one lane per row, a slice's
 // entries column-major so every entry column is one coalesced load, eight
 // columns' loads and gathers in flight per lane; rows too long for a slice are
 // walked by a whole wave from the CSR arrays (lane-strided + butterfly). A
 // row's sum is its entries in CSR order (padding adds fma(0, x[row], s) = s).
 // With want_dot, the partials of x.y go to part as in spmv_pAp.
-template <class VT>
+// WIDE: operators with long rows, sixteen entries of a lane in flight instead
+// of eight, which the 7-entry rows of a grid would pay for in registers (128^3:
+// 64 instead of 54 us). With the long rows walked in pipelined rounds from the
+// mean length on (see the setup), dealt over all bands and first, R-MAT s18
+// (hub row of 25,209 entries) fell from 244 to 86 us, s14 from 50 to 15.
+template <class VT, bool WIDE>
 __device__ __forceinline__ void spmv_sell_body(int vb, int vg, const sell_desc& a, const double* __restrict__ x,
                                                double* __restrict__ y, const pcg_state* st, double* part,
                                                int want_dot) {
@@ -70,55 +161,39 @@ __device__ __forceinline__ void spmv_sell_body(int vb, int vg, const sell_desc& 
     __shared__ double sh[kWavesPerBlock * 2];
     const int lane = threadIdx.x & (kWave - 1);
     // XCD-aware split: the dispatcher places workgroup b on XCD b % kXcds, so
-    // the items (slices, then long rows) are cut into kXcds contiguous bands
-    // and band x is shared by the workgroups b = x (mod kXcds). With slices in
-    // vertex order each XCD's L2 then serves one band of rows and the x
-    // entries they gather. (The grid is a multiple of kXcds; the split only
-    // places work, every item is done once whatever the placement.)
+    // the slices are cut into kXcds contiguous bands and band x is shared by
+    // the workgroups b = x (mod kXcds). With slices in vertex order each XCD's
+    // L2 then serves one band of rows and the x entries they gather. The long
+    // rows (longest first) are dealt to the bands in turn and come before the
+    // band's slices: the hub rows are the longest chains of the launch. (The
+    // grid is a multiple of kXcds; the split only places work, every item is
+    // done once whatever the placement.)
     const int band = vb % kXcds;
     const int per = vg / kXcds;
-    const int items = a.nslices + a.nlong;
-    const int i0 = static_cast<int>(static_cast<long long>(items) * band / kXcds);
-    const int i1 = static_cast<int>(static_cast<long long>(items) * (band + 1) / kXcds);
+    const int nlong = WIDE ? (a.nlong - band + kXcds - 1) / kXcds : 0;
+    const int s0 = static_cast<int>(static_cast<long long>(a.nslices) * band / kXcds);
+    const int items = nlong + static_cast<int>(static_cast<long long>(a.nslices) * (band + 1) / kXcds) - s0;
     const int wave = __builtin_amdgcn_readfirstlane(vb / kXcds * kWavesPerBlock + static_cast<int>(threadIdx.x) / kWave);
     const int* __restrict__ sidx = a.idx;
     const VT* __restrict__ sval = static_cast<const VT*>(a.val);
     double acc = 0.0;
-    for (int it = i0 + wave; it < i1; it += per * kWavesPerBlock) {
-        if (it < a.nslices) {
+    for (int item = wave; item < items; item += per * kWavesPerBlock) {
+        if (!WIDE || item >= nlong) {
+            const int it = s0 + item - nlong;
             const unsigned c0 = a.soff[it], c1 = a.soff[it + 1];
             const int w = static_cast<int>(c1 - c0);
             const size_t base = static_cast<size_t>(c0) * kWave + lane;
             const int row = a.rowmap[static_cast<size_t>(it) * kWave + lane];
-            // Columns in groups of eight (the last group predicated): all of a
-            // group's loads, then its gathers, are in flight together.
-            double s = 0.0;
-            for (int k = 0; k < w; k += 8) {
-                int j[8];
-                double v[8], g[8];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                    const bool ok = k + u < w;
-                    j[u] = ok ? sidx[base + static_cast<size_t>(k + u) * kWave] : 0;
-                    v[u] = ok ? static_cast<double>(sval[base + static_cast<size_t>(k + u) * kWave]) : 0.0;
-                }
-#pragma unroll
-                for (int u = 0; u < 8; ++u) g[u] = k + u < w ? x[j[u]] : 0.0;
-#pragma unroll
-                for (int u = 0; u < 8; ++u)
-                    if (k + u < w) s = fma(v[u], g[u], s);
-            }
+            const double s = slice_sum<WIDE ? 16 : 8, VT>(sidx, sval, base, w, x);
             if (row >= 0 && row < a.n) {
                 y[row] = s;
                 acc = fma(x[row], s, acc);
             }
         } else {
-            const int row = a.longrows[it - a.nslices];
+            const int row = a.longrows[band + item * kXcds];
             const unsigned b = a.ptr[row], e = a.ptr[row + 1];
             const VT* __restrict__ cval = static_cast<const VT*>(a.cval);
-            double s = 0.0;
-            for (unsigned p = b + lane; p < e; p += kWave) s = fma(static_cast<double>(cval[p]), x[a.cidx[p]], s);
-            s = wave_sum(s);
+            const double s = wave_sum(long_row_sum<16, VT>(a.cidx, cval, b, e, lane, [&](int j) { return x[j]; }));
             if (lane == 0) {
                 y[row] = s;
                 acc = fma(x[row], s, acc);
@@ -129,10 +204,10 @@ __device__ __forceinline__ void spmv_sell_body(int vb, int vg, const sell_desc& 
     double v[1] = {acc};
     block_partials<1>(v, part, sh, vb);
 }
-template <class VT>
+template <class VT, bool WIDE>
 __global__ __launch_bounds__(kBlock) void spmv_sell(sell_desc a, const double* __restrict__ x, double* __restrict__ y,
                                                     const pcg_state* st, double* part, int want_dot) {
-    spmv_sell_body<VT>(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), a, x, y, st, part, want_dot);
+    spmv_sell_body<VT, WIDE>(static_cast<int>(blockIdx.x), static_cast<int>(gridDim.x), a, x, y, st, part, want_dot);
 }
 
 // r[perm[v]] = b[v]; x[perm[v]] = x0[v] (or 0).
