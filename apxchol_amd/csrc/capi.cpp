@@ -819,7 +819,9 @@ apx_status apx_solve(int64_t n, const int64_t* colptr, const int32_t* rowidx, co
     return guarded([&] {
         const csc_view A = make_view(n, colptr, rowidx, vals);
         if (n > 0) { need(b, "b"); need(x, "x"); }
-        const gpu_solver slv(A, to_opts(opts));
+        solve_options o = to_opts(opts);
+        o.merge_levels = false;   // one solve does not repay the setup
+        const gpu_solver slv(A, o);
         solve_result r = slv.solve(std::vector<double>(b, b + n));
         if (n > 0) std::memcpy(x, r.x.data(), static_cast<std::size_t>(n) * sizeof(double));
         fill_info(r, info);

@@ -184,6 +184,23 @@ struct trail_desc {
     const int4* longrow = nullptr;
 };
 
+// Merged levels (kernels/merge.hip): a batch of up to 64 lanes whose rows are
+// sums over earlier outputs and right-hand sides. Lane l of batch b works for
+// rec[b * 64 + l].row (info: log2 G | sub << 3 | entries << 9); its entry k is
+// slot ((chunk + k / kEpl) * kEpl + k % kEpl) * 64 + l of idx / val. idx >= 0:
+// the output of that row; idx < 0: the right-hand side of row ~idx.
+struct alignas(8) merge_batch {
+    std::uint32_t chunk;    // first chunk of kEpl * 64 slots
+    std::uint32_t chunks;
+};
+struct merge_desc {
+    const lane_rec* rec = nullptr;
+    const merge_batch* batch = nullptr;
+    const std::int32_t* idx = nullptr;
+    const double* val = nullptr;
+    int batches = 0;
+};
+
 // Per (tail batch, lane), written by the coupling kernel before a run: the
 // lane's fma chain over the entries before the run, and the row's right-hand
 // side (writer lanes).

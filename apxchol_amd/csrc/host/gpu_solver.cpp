@@ -17,9 +17,11 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
+#include <thread>
 
 #include "../device.hpp"
 #include "../kernels/launch.hpp"
+#include "merge.hpp"
 #include "trail.hpp"
 
 namespace apxchol_amd {
@@ -527,6 +529,9 @@ struct gpu_solver::device_state {
     // The trailing block (t.n == 0: none), its product's input and layouts.
     trail_desc trail;
     dbuf tr_s, tr_c, tr_rec, tr_ent, tr_long;
+    // The merged levels outside it, per direction.
+    std::vector<merge_step> plan[2];
+    dbuf mg_rec[2], mg_batch[2], mg_idx[2], mg_val[2];
     dbuf part, st, st_apply, ctrl, err;
     pcg_state* host_st = nullptr;
     int* host_err = nullptr;
@@ -1174,6 +1179,61 @@ void gpu_solver::setup(const csc_view& L) {
                d.f_level_pos, d.f_level_diag);
     make_sched(d.b_sched, bb, true, d.b_levels, d.b_levels_dev, d.b_seg, b_tb, d.b_level_lb, d.b_lrec, d.b_lent,
                d.b_level_pos, d.b_level_diag);
+    // An application's steps outside the trailing block, the two directions side
+    // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
+    // may gain; 0: no merging).
+    long long growth = opts_.merge_levels ? -1 : 0;
+    if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
+    if (d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0) {
+        const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
+        merge_tables mt[2];
+        std::exception_ptr failed;
+        std::thread back([&] {
+            try {
+                mt[1] = build_merged_levels(T_, true, L - c, L, d.b_levels, growth);
+            } catch (...) {
+                failed = std::current_exception();
+            }
+        });
+        try {
+            mt[0] = build_merged_levels(T_, false, 0, c, d.f_levels, growth);
+        } catch (...) {
+            back.join();
+            throw;
+        }
+        back.join();
+        if (failed) std::rethrow_exception(failed);
+        for (int dir = 0; dir < 2; ++dir) {
+            merge_tables& t = mt[dir];
+            d.plan[dir] = t.steps;
+            d.mg_rec[dir].upload(t.rec);
+            d.mg_batch[dir].upload(t.batch);
+            d.mg_idx[dir].alloc(t.slots * sizeof(std::int32_t));
+            d.mg_val[dir].alloc(t.slots * sizeof(double));
+            std::size_t at = 0;
+            for (const auto& q : t.pieces) {
+                hip_check(hipMemcpy(d.mg_idx[dir].as<std::int32_t>() + at, q.idx.data(),
+                                    q.idx.size() * sizeof(std::int32_t), hipMemcpyHostToDevice), "upload");
+                hip_check(hipMemcpy(d.mg_val[dir].as<double>() + at, q.val.data(), q.val.size() * sizeof(double),
+                                    hipMemcpyHostToDevice), "upload");
+                at += q.idx.size();
+            }
+            sweep_sched& sc = dir ? d.b_sched : d.f_sched;
+            sc.planned = true;
+            sc.plan = d.plan[dir].data();
+            sc.nplan = static_cast<int>(d.plan[dir].size());
+            sc.merged.rec = d.mg_rec[dir].as<lane_rec>();
+            sc.merged.batch = d.mg_batch[dir].as<merge_batch>();
+            sc.merged.idx = d.mg_idx[dir].as<std::int32_t>();
+            sc.merged.val = d.mg_val[dir].as<double>();
+            sc.merged.batches = static_cast<int>(t.batch.size());
+            // An application launches its steps, no tail runs.
+            stats_.solve_level_bytes[dir] += stats_.solve_tail_bytes[dir];
+            stats_.solve_tail_bytes[dir] = 0;
+            stats_.solve_tail_runs[dir] = 0;
+            stats_.solve_level_launches[dir] = sc.nplan;
+        }
+    }
     // Coupling output, shared by the two directions (their sweeps never overlap).
     const std::size_t tail_batches = std::max<std::size_t>(
         1, static_cast<std::size_t>(std::max(d.f_sched.tail_batches, d.b_sched.tail_batches)));
@@ -1205,7 +1265,9 @@ void gpu_solver::setup(const csc_view& L) {
                           &d.op_val, &d.r, &d.x, &d.p, &d.ap, &d.rp, &d.y, &d.z, &d.xout, &d.f_lrec, &d.f_lent,
                           &d.b_lrec, &d.b_lent, &d.f_tlane, &d.f_tent, &d.f_tovf, &d.f_tovf_ent, &d.f_twalk,
                           &d.b_tlane, &d.b_tent, &d.b_tovf, &d.b_tovf_ent, &d.b_twalk, &d.f_tlane_r, &d.b_tlane_r,
-                          &d.tail_val, &d.relabel, &d.tr_s, &d.tr_c, &d.tr_rec, &d.tr_ent, &d.tr_long, &d.sell_soff,
+                          &d.tail_val, &d.relabel, &d.tr_s, &d.tr_c, &d.tr_rec, &d.tr_ent, &d.tr_long,
+                          &d.mg_rec[0], &d.mg_batch[0], &d.mg_idx[0], &d.mg_val[0], &d.mg_rec[1], &d.mg_batch[1],
+                          &d.mg_idx[1], &d.mg_val[1], &d.sell_soff,
                           &d.sell_idx, &d.sell_val, &d.sell_map, &d.sell_long})
         bytes += b->bytes();
     stats_.device_bytes = bytes;
@@ -1661,6 +1723,7 @@ const block_sched* gpu_solver::block_scheds(int kp, int which) const {
                 l = e;
             }
             if (cl == nl) sc.cut_seg = static_cast<int>(seg[0].size());
+            sc.merged = backward ? &dev_->b_sched : &dev_->f_sched;
             sc.kp = kp;
             sc.pos = dp.as<unsigned>();
             sc.mask = dm.as<unsigned long long>();
@@ -2149,6 +2212,54 @@ group_member_view gpu_solver::group_view() const {
         const sweep_desc& desc = dir ? d.bck : d.fwd;
         if (desc.nb == 0) continue;
         if (sc.kind != 2) throw std::invalid_argument("gpu_solver::group: a group member's sweeps must be the hybrid schedule");
+        const auto level_unit = [&](int l) {
+            group_unit u;
+            u.d = desc;
+            u.b0 = sc.level_first[l];
+            u.b1 = sc.level_first[l + 1];
+            if (u.b1 <= u.b0) return;
+            u.rhs = dir ? d.y.get() : d.r.get();
+            u.out = dir ? d.z.get() : d.y.get();
+            u.err = d.err.as<int>();
+            const int lb = sc.level_lb ? sc.level_lb[l] : -1;
+            if (lb >= 0) {
+                u.kind = kGroupLane;
+                u.lb0 = lb;
+                u.nlb = u.b1 - u.b0;
+                u.rec = sc.lane_rec_dev;
+                u.ent = sc.lane_ent_dev;
+                if (static_cast<long long>(lb) + u.nlb > sc.lane_batches)
+                    throw std::runtime_error("gpu_solver::group: level outside the lane layout");
+                u.grid = (u.nlb + kLevelWavesPerBlock - 1) / kLevelWavesPerBlock;
+            } else {
+                u.kind = kGroupLevels;
+                u.grid = std::min((u.b1 - u.b0 + kLevelWavesPerBlock - 1) / kLevelWavesPerBlock, kLevelLaunchMaxBlocks);
+            }
+            v.steps[dir].push_back(u);
+        };
+        if (sc.planned) {
+            for (int k = 0; k < sc.nplan; ++k) {
+                const merge_step& t = sc.plan[k];
+                if (t.nb == 0) {
+                    for (int l = t.l0; l < t.l1; ++l) level_unit(l);
+                    continue;
+                }
+                group_unit u;
+                u.kind = kGroupMerged;
+                u.d = desc;
+                u.mg = sc.merged;
+                u.lb0 = t.b0;
+                u.nlb = t.nb;
+                u.rhs = dir ? d.y.get() : d.r.get();
+                u.out = dir ? d.z.get() : d.y.get();
+                u.err = d.err.as<int>();
+                u.grid = (t.nb + kLevelWavesPerBlock - 1) / kLevelWavesPerBlock;
+                if (t.b0 < 0 || t.b0 + t.nb > sc.merged.batches)
+                    throw std::runtime_error("gpu_solver::group: merged step outside its layout");
+                v.steps[dir].push_back(u);
+            }
+            continue;
+        }
         const bool block = d.trail.n > 0;
         const int k0 = block && dir ? sc.cut_seg : 0, k1 = block && !dir ? sc.cut_seg : sc.nseg;
         for (int k = k0; k < k1; ++k) {
@@ -2175,31 +2286,7 @@ group_member_view gpu_solver::group_view() const {
                 v.steps[dir].push_back(u);
                 continue;
             }
-            for (int l = sc.seg_l0[k]; l < sc.seg_l1[k]; ++l) {
-                group_unit u;
-                u.d = desc;
-                u.b0 = sc.level_first[l];
-                u.b1 = sc.level_first[l + 1];
-                if (u.b1 <= u.b0) continue;
-                u.rhs = dir ? d.y.get() : d.r.get();
-                u.out = dir ? d.z.get() : d.y.get();
-                u.err = d.err.as<int>();
-                const int lb = sc.level_lb ? sc.level_lb[l] : -1;
-                if (lb >= 0) {
-                    u.kind = kGroupLane;
-                    u.lb0 = lb;
-                    u.nlb = u.b1 - u.b0;
-                    u.rec = sc.lane_rec_dev;
-                    u.ent = sc.lane_ent_dev;
-                    if (static_cast<long long>(lb) + u.nlb > sc.lane_batches)
-                        throw std::runtime_error("gpu_solver::group: level outside the lane layout");
-                    u.grid = (u.nlb + kLevelWavesPerBlock - 1) / kLevelWavesPerBlock;
-                } else {
-                    u.kind = kGroupLevels;
-                    u.grid = std::min((u.b1 - u.b0 + kLevelWavesPerBlock - 1) / kLevelWavesPerBlock, kLevelLaunchMaxBlocks);
-                }
-                v.steps[dir].push_back(u);
-            }
+            for (int l = sc.seg_l0[k]; l < sc.seg_l1[k]; ++l) level_unit(l);
         }
     }
     return v;

@@ -38,6 +38,7 @@ struct solve_options {
     int sweep_chunk = 0;          // batches per dataflow ticket (0: APXCHOL_AMD_SWEEP_CHUNK or 8)
     int sweep_blocks = 0;         // dataflow grid (0: APXCHOL_AMD_SWEEP_BLOCKS or the resident grid)
     bool graph = true;            // replay each PCG iteration as one captured HIP graph
+    bool merge_levels = true;     // merge levels outside the trailing block (off for one-shot solves)
     bool relabel = true;          // sort every level's rows by original vertex (APXCHOL_AMD_RELABEL=0: off)
     bool depth_levels = true;     // with relabel: levels = topological depth (APXCHOL_AMD_DEPTH_LEVELS=0: rounds)
     int lane_batches = 0;         // launched levels of <= this many batches use the lane layout

@@ -121,6 +121,9 @@ __global__ __launch_bounds__(kBlock) void group_sweep_level(const group_unit* __
     if (u.kind == kGroupLane)
         sweep_lanes_body<TI, TO, F16>(vb, u.d, u.lb0, u.nlb, u.rec, u.ent, static_cast<const TI*>(u.rhs),
                                       static_cast<TO*>(u.out), u.st);
+    else if (sizeof(TO) == sizeof(double) && u.kind == kGroupMerged)
+        sweep_merged_body<1>(vb, 0, u.mg, u.lb0, u.nlb, u.d.backward, static_cast<const double*>(u.rhs),
+                             static_cast<double*>(u.out), u.st, 1, nullptr);
     else
         sweep_levels_body<TI, TO, F16>(vb, starts[i + 1] - starts[i], u.d, u.b0, u.b1, static_cast<const TI*>(u.rhs),
                                        static_cast<TO*>(u.out), u.st, u.err);

@@ -14,6 +14,7 @@
 #include "sweep.hip"
 #include "block.hip"
 #include "trail.hip"
+#include "merge.hip"
 #include "pieces.hip"
 #include "group.hip"
 
@@ -61,6 +62,11 @@ int dataflow_grid_for() {
         per_cu <= 0)
         per_cu = 1;
     return per_cu * cus;
+}
+
+void check_merged(const sweep_sched& sc, const merge_step& t) {
+    if (t.b0 < 0 || t.nb < 0 || t.b0 + t.nb > sc.merged.batches)
+        throw std::runtime_error("apxchol_amd: merged step outside its layout");
 }
 
 // Workgroups of one level launch: one wave per batch, up to this many.
@@ -111,7 +117,21 @@ void sweep_t(const sweep_desc& d, const void* rhs, void* out, const pcg_state* s
         if (g > kLevelMaxBlocks) g = kLevelMaxBlocks;
         launch_timed(hook, 0, sweep_levels<TI, TO, F16>, dim3(g), dim3(kBlock), 0, s, d, b0, b1, in, o, st, err);
     };
-    if (sc.kind == 0) {
+    if (outside && sc.planned) {   // fp64 vectors
+        for (int k = 0; k < sc.nplan; ++k) {
+            const merge_step& t = sc.plan[k];
+            if (t.nb == 0) {
+                for (int l = t.l0; l < t.l1; ++l) level_launch(l);
+                continue;
+            }
+            check_merged(sc, t);
+            launch_timed(hook, 0, sweep_merged<1>,
+                         dim3(static_cast<unsigned>((t.nb + kWavesPerBlock - 1) / kWavesPerBlock)), dim3(kBlock), 0, s,
+                         sc.merged, t.b0, t.nb, static_cast<int>(d.backward), static_cast<const double*>(rhs),
+                         static_cast<double*>(out), st, 1, static_cast<const batch_state*>(nullptr));
+        }
+        check_launch("sweep_merged");
+    } else if (sc.kind == 0) {
         sweep_desc part = d;
         range(sc.cut_batch, d.nb, part.b_first, part.nb);
         if (part.b_first >= part.nb) return;
@@ -544,7 +564,29 @@ void sweep_k_t(const sweep_desc& d, const block_sched& b, const void* rhs, void*
         sweep_block<TI, TO, F16><<<g, kBlock, 0, s>>>(d, b.pos, b.mask, b.col0, w0, w1, b.kp,
                                                       static_cast<const TI*>(rhs), static_cast<TO*>(out), st, bs);
     };
-    if (b.cols) {
+    if (outside && b.merged && b.merged->planned) {
+        // Columns per wave: the operands of an entry for 4 columns are two
+        // 16-byte loads.
+        const sweep_sched& sc = *b.merged;
+        const double* in = static_cast<const double*>(rhs);
+        double* o = static_cast<double*>(out);
+        const int cb = std::min(b.kp, 4);
+        for (int k = 0; k < sc.nplan; ++k) {
+            const merge_step& t = sc.plan[k];
+            if (t.nb == 0) {
+                for (int l = t.l0; l < t.l1; ++l) level_launch(l);
+                continue;
+            }
+            check_merged(sc, t);
+            const dim3 g(static_cast<unsigned>((t.nb + kWavesPerBlock - 1) / kWavesPerBlock), static_cast<unsigned>(b.kp / cb));
+            auto go = [&](auto kernel) {
+                kernel<<<g, kBlock, 0, s>>>(sc.merged, t.b0, t.nb, static_cast<int>(d.backward), in, o, st, b.kp, bs);
+            };
+            if (cb == 1) go(sweep_merged<1>);
+            else if (cb == 2) go(sweep_merged<2>);
+            else go(sweep_merged<4>);
+        }
+    } else if (b.cols) {
         // The single-vector schedule, column by column: its launched levels
         // as blocked level launches, each of its tail runs as one coupling
         // launch over (batch, column) and one tail workgroup per column.

@@ -18,6 +18,14 @@ bool sweep_tail_fits(vec_prec p, int rows, int batches, int levels);
 // LDS bytes of the walk of a tail run of `rows` rows and `batches` batches.
 std::size_t sweep_tail_lds(vec_prec p, int rows, int batches);
 
+// One step of an application's sweep over the levels outside the trailing
+// block: levels [l0, l1) (in sweep order). A step of one level is launched as
+// that level; a longer one as the merged batches [b0, b0 + nb).
+struct merge_step {
+    int l0 = 0, l1 = 0;
+    int b0 = 0, nb = 0;
+};
+
 // How one sweep direction is scheduled.
 //   dataflow: one persistent launch of `grid` workgroups (polling);
 //   levels:   one launch per level;
@@ -59,6 +67,13 @@ struct sweep_sched {
     // The boundary of the trailing block in this direction: its first level,
     // segment and batch (back sweep: the first ones after it).
     int cut_level = 0, cut_seg = 0, cut_batch = 0;
+    // How an application covers the levels outside the block, in every kind of
+    // schedule (host; planned: there is a block): steps of one launch each, a
+    // level or merged levels.
+    bool planned = false;
+    const merge_step* plan = nullptr;
+    int nplan = 0;
+    merge_desc merged;
 };
 // The rows a sweep launch covers: all, or those outside the trailing block
 // (the back sweep then expects the block's outputs in place).
@@ -164,6 +179,7 @@ struct block_sched {
     const int* seg_tail = nullptr;
     int nseg = 0;
     int cut_level = 0, cut_seg = 0;         // the trailing block's boundary, as in sweep_sched
+    const sweep_sched* merged = nullptr;    // the schedule whose plan an application follows
     // When set: the single-vector schedule whose levels this sweep follows,
     // its tail runs walked column by column (one tail workgroup per column)
     // with the coupling values in col_tail_val (kp * 64 tail_val per run batch).
@@ -229,7 +245,7 @@ struct group_member {
     const int* oidx = nullptr;
     const void* oval = nullptr;
 };
-inline constexpr int kGroupLane = 0, kGroupLevels = 1, kGroupTail = 2;
+inline constexpr int kGroupLane = 0, kGroupLevels = 1, kGroupTail = 2, kGroupMerged = 3;
 // One member's trailing block in a grouped launch.
 struct group_trail {
     trail_desc t;
@@ -251,6 +267,7 @@ struct group_unit {
     const lane_rec* rec = nullptr;
     const entry32* ent = nullptr;
     int b0 = 0, b1 = 0;                     // batch-table level / tail run: batches [b0, b1)
+    merge_desc mg;                          // merged levels: lane batches [lb0, lb0 + nlb) of it
     int p0 = 0;                             // tail run: its first sweep position
     tail_desc td;                           // tail run: the direction's tail layout
     int base = 0, nlev = 0, zslot = 0, row0 = 0;

@@ -74,6 +74,58 @@ def test_block_rows_match_oracle_and_all_paths_agree(gpu, name, rows, monkeypatc
         s.close()
 
 
+@pytest.mark.parametrize("name", list(CASES))
+@pytest.mark.parametrize("growth", [0, 1, 300, 4000, 10_000_000])
+def test_merged_levels_match_oracle_and_all_paths_agree(gpu, name, growth, monkeypatch):
+    """The levels outside the block, merged from not at all to all into one
+    launch (rows of several chunks of 256 entries)."""
+    import torch
+    print(f"[case] merged levels {name} growth={growth}", flush=True)
+    A, F, fac = case(name)
+    monkeypatch.setenv("APXCHOL_AMD_TRAIL_ROWS", "64")
+    monkeypatch.setenv("APXCHOL_AMD_MERGE_GROWTH", str(growth))
+    R = np.random.default_rng(growth % 97).standard_normal((6, A.shape[0]))
+    Rd = torch.tensor(R, device=gpu)
+    solvers = []
+    for precision, fp16 in (("fp64", False), ("fp32", False), ("fp64", True), ("fp32", True)):
+        s = ax.Solver(A, factor=F, precision=precision, fp16_storage=fp16)
+        blk = s.info["block"]
+        assert 0 < blk["rows"] <= 64
+        if growth > 0 and precision == "fp64":
+            assert blk["tail_runs"] == [0, 0]
+        if growth == 10_000_000 and precision == "fp64":
+            assert max(blk["level_launches"]) < 0.5 * s.info["levels"]
+        s.reset_apply_count()
+        Z = s.apply_batch(Rd).cpu().numpy()
+        tol = 1e-12 if precision == "fp64" else 1e-5 if fp16 else 1e-6
+        for c in range(6):
+            s.reset_apply_count()
+            z = s.apply(Rd[c].clone()).cpu().numpy()
+            assert np.array_equal(bits(z), bits(Z[c])), (precision, fp16, c)
+            if c < 2:
+                ref = oracle.Oracle(A, fac, F.sddm, fp16=fp16).apply(R[c])
+                err = np.max(np.abs(z - ref)) / np.max(np.abs(ref))
+                assert err < tol, (precision, fp16, c, err)
+        for schedule in ("levels", "dataflow"):
+            o = ax.Solver(A, factor=F, precision=precision, fp16_storage=fp16, schedule=schedule)
+            z = o.apply(Rd[0].clone()).cpu().numpy()
+            assert np.array_equal(bits(z), bits(Z[0])), (precision, fp16, schedule)
+            o.close()
+        if not fp16:
+            solvers.append((precision, s))
+        else:
+            s.close()
+    b = torch.tensor(mg.request_rhs(A, F.sddm, 5), device=gpu)
+    for precision, s in solvers:
+        one = ax.Group([s])
+        xs, rs = one.solve([b], tol=1e-8, maxiter=200)
+        own = s.solve(b, tol=1e-8, maxiter=200)
+        torch.cuda.synchronize()
+        assert rs[0].status == 1 and torch.equal(xs[0].view(torch.int64), own.x.view(torch.int64)), precision
+        one.close()
+        s.close()
+
+
 @pytest.mark.parametrize("precision", ["fp64", "fp32"])
 @pytest.mark.parametrize("k", [1, 2, 8, 17, 33, 64])
 def test_block_columns_have_the_single_bits(gpu, precision, k):
