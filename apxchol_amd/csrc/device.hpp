@@ -88,6 +88,10 @@ struct pcg_state {
     int pad_i;
 };
 
+// Partials a column of a blocked reduction may have: the vector kernels' grid
+// cap (2048), the SpMM's rounding up and the long rows' one more.
+inline constexpr int kColPartials = 2080;
+
 // Bookkeeping of a blocked (k right-hand sides) solve: the number of columns
 // still iterating; every blocked kernel returns at once when it is zero.
 struct batch_state {

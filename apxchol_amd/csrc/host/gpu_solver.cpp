@@ -1555,9 +1555,8 @@ int gpu_solver::prepare_block(int k, int which) const {
     b.c.alloc(static_cast<std::size_t>(dev_->trail.n) * kp * sizeof(double));
     b.st.alloc(static_cast<std::size_t>(kp) * sizeof(pcg_state));
     b.bs.alloc(sizeof(batch_state));
-    // Partials: 2 values x kp columns per workgroup; the SpMM grid may round
-    // kMaxBlocksHost up by at most 15 (a multiple of G kp / 256 <= 16).
-    b.part.alloc(static_cast<std::size_t>(kMaxBlocksHost + 16) * 2 * kp * sizeof(double));
+    // Partials: 2 values x kp columns per workgroup.
+    b.part.alloc(static_cast<std::size_t>(kColPartials) * 2 * kp * sizeof(double));
     if (b.host_st) (void)hipHostFree(b.host_st);
     b.host_st = nullptr;
     hip_check(hipHostMalloc(reinterpret_cast<void**>(&b.host_st), static_cast<std::size_t>(kp) * sizeof(pcg_state),

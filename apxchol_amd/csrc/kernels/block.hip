@@ -278,9 +278,16 @@ __global__ __launch_bounds__(kTailBlock) void sweep_block_tail(sweep_desc d, con
 
 // ---- per-column reductions -----------------------------------------------
 
+// Slot of producer workgroup `block`'s partial k of column c: a column's
+// partials lie side by side for block_finish.
+inline constexpr int kFinishMaxBlocks = kColPartials;
+__device__ __forceinline__ size_t col_part(int block, int k, int c, int kp) {
+    return static_cast<size_t>(k * kp + c) * kFinishMaxBlocks + block;
+}
+
 // Two-stage per-column reductions (kp columns, kBlock / kp rows per block),
 // as block_partials / finish_sum for one vector. Stage 1: the block's column
-// sums, in row order, to part[(block * N + k) * kp + j].
+// sums, in row order, to part[col_part(block, k, j, kp)].
 //
 // Lane mapping: thread t of the grid serves column ((t / G) % kp) and only
 // its chain-0 lanes (t % G == 0) carry values (the others hold exact zeros,
@@ -304,47 +311,69 @@ __device__ __forceinline__ void col_block_partials(double (&v)[N], int kp, doubl
                 const int off = (c - first + kp) % kp;
                 if (off < kBlock / G) s = sh[k * kBlock + off * G];
             }
-            part[(static_cast<size_t>(blockIdx.x) * N + k) * kp + c] = s;
+            part[col_part(static_cast<int>(blockIdx.x), k, c, kp)] = s;
         }
     }
 }
 
-// Stage 2 (one workgroup) over the partials of nb blocks: thread (j, c) sums
-// blocks j, j + rows, ... of column c (eight loads in flight at a time), then
-// column c's `rows` sums are added in j order. Thread c < kp returns true
-// with the totals of column c in v.
+// Stage 2 over the partials of nb blocks, workgroup c for column c: kBlock / kp
+// chains, chain j over the blocks j, j + kBlock / kp, ..., added in j order.
+// All threads bring the column's partials to LDS in one round of loads; the
+// chains then run from there (one workgroup for all columns with eight loads
+// a chain in flight took 18.6 us at 2,048 blocks x 32 columns; 8.1 now). Thread 0
+// returns true with the totals in v.
 template <int N>
 __device__ __forceinline__ bool col_finish_sum(double (&v)[N], int kp, const double* part, int nb, double* sh) {
-    const int c = threadIdx.x & (kp - 1);
+    const int c = static_cast<int>(blockIdx.x);
     const int rows = kBlock / kp;
-    const int j = threadIdx.x / kp;
+    constexpr int U = (kFinishMaxBlocks + kBlock - 1) / kBlock;
+    double g[U][N];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int b = static_cast<int>(threadIdx.x) + u * kBlock;
+        if (b < nb)
+#pragma unroll
+            for (int k = 0; k < N; ++k) g[u][k] = part[col_part(b, k, c, kp)];
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const int b = static_cast<int>(threadIdx.x) + u * kBlock;
+        if (b < nb)
+#pragma unroll
+            for (int k = 0; k < N; ++k) sh[k * kFinishMaxBlocks + b] = g[u][k];
+    }
+    __syncthreads();
+    const int j = static_cast<int>(threadIdx.x);
     double acc[N];
 #pragma unroll
     for (int k = 0; k < N; ++k) acc[k] = 0.0;
-    // Eight blocks' loads in flight at once, added in block order.
-    int b = j;
-    for (; b + 7 * rows < nb; b += 8 * rows) {
-        double g[8][N];
+    if (j < rows) {
+        int b = j;
+        for (; b + 7 * rows < nb; b += 8 * rows) {
+            double q[8][N];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < 8; ++u)
 #pragma unroll
-            for (int k = 0; k < N; ++k) g[u][k] = part[(static_cast<size_t>(b + u * rows) * N + k) * kp + c];
+                for (int k = 0; k < N; ++k) q[u][k] = sh[k * kFinishMaxBlocks + b + u * rows];
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
+            for (int u = 0; u < 8; ++u)
 #pragma unroll
-            for (int k = 0; k < N; ++k) acc[k] += g[u][k];
+                for (int k = 0; k < N; ++k) acc[k] += q[u][k];
+        }
+        for (; b < nb; b += rows)
+#pragma unroll
+            for (int k = 0; k < N; ++k) acc[k] += sh[k * kFinishMaxBlocks + b];
     }
-    for (; b < nb; b += rows)
-#pragma unroll
-        for (int k = 0; k < N; ++k) acc[k] += part[(static_cast<size_t>(b) * N + k) * kp + c];
-#pragma unroll
-    for (int k = 0; k < N; ++k) sh[k * kBlock + threadIdx.x] = acc[k];
     __syncthreads();
-    if (threadIdx.x >= kp) return false;
+    if (j < rows)
+#pragma unroll
+        for (int k = 0; k < N; ++k) sh[k * kBlock + j] = acc[k];
+    __syncthreads();
+    if (threadIdx.x != 0) return false;
 #pragma unroll
     for (int k = 0; k < N; ++k) {
-        double s = sh[k * kBlock + c];
-        for (int i = 1; i < rows; ++i) s += sh[k * kBlock + i * kp + c];
+        double s = sh[k * kBlock];
+        for (int i = 1; i < rows; ++i) s += sh[k * kBlock + i];
         v[k] = s;
     }
     return true;
@@ -600,7 +629,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_dot_k(sell_desc a, int kp, c
     if (threadIdx.x < kp) {
         double t = sh[c];
         for (int r = 1; r < rows; ++r) t += sh[r * kp + c];
-        part[static_cast<size_t>(nb) * kp + c] = t;
+        part[col_part(nb, 0, c, kp)] = t;
     }
 }
 
@@ -793,8 +822,8 @@ __global__ __launch_bounds__(kBlock) void sum_cols_k(int n, int kp, const T* __r
     col_block_partials<1>(v, kp, part, sh);
 }
 
-// Stage 2 of the blocked reductions (one workgroup, launched right after the
-// producer of `part`; nb = the producer's grid), per column c < kp:
+// Stage 2 of the blocked reductions (one workgroup per column, launched right
+// after the producer of `part`; nb = the producer's grid), per column c < kp:
 //   kBFinPAp        st[c].pAp of an iterating column; breakdown ends it
 //   kBFinInit       start of each joining column (init_residual's decisions)
 //   kBFinXR         each live column's loop bookkeeping (update_xr's)
@@ -806,7 +835,7 @@ enum : int { kBFinPAp, kBFinInit, kBFinXR, kBFinDot, kBFinDotFirst, kBFinOutSum 
 __global__ __launch_bounds__(kBlock) void block_finish(int op, int n, int kp, const double* __restrict__ part, int nb,
                                                        pcg_state* st, const batch_state* bs) {
     if ((op == kBFinPAp || op == kBFinXR || op == kBFinDot || op == kBFinDotFirst) && bs->active == 0) return;
-    __shared__ double sh[2 * kBlock];
+    __shared__ double sh[2 * kFinishMaxBlocks];
     double v[2] = {0.0, 0.0};
     bool mine;
     if (op == kBFinPAp || op == kBFinOutSum) {
@@ -817,7 +846,7 @@ __global__ __launch_bounds__(kBlock) void block_finish(int op, int n, int kp, co
         mine = col_finish_sum<2>(v, kp, part, nb, sh);
     }
     if (!mine) return;
-    pcg_state& t = st[threadIdx.x];
+    pcg_state& t = st[blockIdx.x];
     switch (op) {
         case kBFinPAp:
             if (!t.done && t.phase == 0) {

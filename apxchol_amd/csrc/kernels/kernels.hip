@@ -656,7 +656,8 @@ void check_kp(int kp) {
 
 // Stage 2 of a blocked reduction over the partials of an nb-workgroup producer.
 void finish_k(int op, int n, int kp, const double* part, int nb, pcg_state* st, const batch_state* bs, hipStream_t s) {
-    block_finish<<<1, kBlock, 0, s>>>(op, n, kp, part, nb, st, bs);
+    if (nb > kFinishMaxBlocks) throw std::runtime_error("apxchol_amd: more partials than block_finish holds");
+    block_finish<<<kp, kBlock, 0, s>>>(op, n, kp, part, nb, st, bs);
     check_launch("block_finish");
 }
 
