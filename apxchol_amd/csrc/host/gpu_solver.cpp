@@ -11,6 +11,7 @@
 #include <chrono>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdlib>
 #include <map>
 #include <mutex>
@@ -1406,6 +1407,12 @@ void gpu_solver::enqueue_iteration(int it, hipStream_t s) const {
     enqueue_precondition(false, it, s);
 }
 
+int iterations_ahead(int least, double residual, std::int64_t iterations, double tol) {
+    if (!(residual > tol) || !(residual < 1.0) || !(tol > 0.0) || iterations < 1) return least;
+    const double left = std::log(tol / residual) / std::log(residual) * static_cast<double>(iterations);
+    return std::max(least, static_cast<int>(std::min(0.5 * left, 32.0)));
+}
+
 solve_result gpu_solver::solve_device(const double* d_b, double* d_x, double tol, int max_iter, const double* d_x0,
                                       hipStream_t s) const {
     not_serving("solve");
@@ -1419,8 +1426,12 @@ solve_result gpu_solver::solve_device(const double* d_b, double* d_x, double tol
     single_begin(d_b, d_x0, tol, max_iter, s);
     const int J = std::max(1, opts_.iters_per_check);
     session_slot state;
-    do single_step(J, s);
-    while (!single_poll(state, s));
+    int step = J;
+    for (;;) {
+        single_step(step, s);
+        if (single_poll(state, s)) break;
+        step = iterations_ahead(J, state.residual, state.iterations, tol);
+    }
     single_collect(d_x, res, s);
     res.timings.pcg_ms = ms_since(t_solve);
     std::size_t fr = 0, tot = 0;
@@ -2033,13 +2044,20 @@ std::vector<solve_result> gpu_solver::solve_block(int k, const double* d_B, doub
     launch_init_residual_k(n, kp, b.r.as<double>(), st, bs, b.part.as<double>(), s);
     launch_refresh_active_k(kp, st, bs, s);
     const int J = std::max(1, opts_.iters_per_check);
-    int enqueued = 0;
+    int enqueued = 0, step = J;
     for (;;) {
-        replay_iterations_k(kp, J, s);
-        enqueued += J;
+        replay_iterations_k(kp, step, s);
+        enqueued += step;
         hip_check(hipMemcpyAsync(b.host_bs, bs, sizeof(batch_state), hipMemcpyDeviceToHost, s), "state read");
+        hip_check(hipMemcpyAsync(b.host_st, st, static_cast<std::size_t>(kp) * sizeof(pcg_state), hipMemcpyDeviceToHost, s),
+                  "state read");
         hip_check(hipStreamSynchronize(s), "solve");
-        if (b.host_bs->active == 0 || enqueued > max_iter + J + 1) break;
+        if (b.host_bs->active == 0 || enqueued > max_iter + step + 1) break;
+        // The block runs until its last column is done.
+        step = J;
+        for (int c = 0; c < kp; ++c)
+            if (!b.host_st[c].done)
+                step = std::max(step, iterations_ahead(J, b.host_st[c].residual, b.host_st[c].iter, tol));
     }
     if (!F_.sddm)
         launch_sum_cols_k(vec_prec::fp64, n, kp, b.x.get(), st, b.part.as<double>(), s);

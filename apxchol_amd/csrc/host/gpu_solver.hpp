@@ -100,6 +100,12 @@ struct solver_stats {
 
 struct block_sched;
 
+// Iterations to enqueue before the next completion test: at least `least`,
+// else half of those that the mean convergence so far says are left. A test
+// drains the device (a copy, a wake-up and the next graph launch, about 10 us),
+// and an iteration past the end costs its launches, which return at once.
+int iterations_ahead(int least, double residual, std::int64_t iterations, double tol);
+
 // What a grouped solve (solver_group) needs of one member solver: its device
 // arrays, its solve-state defaults and the steps of its two sweeps (launched
 // levels and tail runs, in order; host copies of the device descriptors).

@@ -271,16 +271,20 @@ std::vector<solve_result> solver_group::solve(const std::vector<const double*>& 
         check(hipGraphInstantiate(&P.exec, P.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
     const int J = 2;
-    int enqueued = 0;
+    int enqueued = 0, step = J;
     for (;;) {
-        for (int j = 0; j < J; ++j) check(hipGraphLaunch(P.exec, s), "hipGraphLaunch");
-        enqueued += J;
+        for (int j = 0; j < step; ++j) check(hipGraphLaunch(P.exec, s), "hipGraphLaunch");
+        enqueued += step;
         check(hipMemcpyAsync(P.host_st, st, static_cast<std::size_t>(N) * sizeof(pcg_state), hipMemcpyDeviceToHost, s),
               "state read");
         check(hipStreamSynchronize(s), "solve");
         bool all = true;
         for (int i = 0; i < N; ++i) all = all && P.host_st[i].done;
-        if (all || enqueued > max_iter + J) break;
+        if (all || enqueued > max_iter + step) break;
+        step = J;
+        for (int i = 0; i < N; ++i)
+            if (!P.host_st[i].done)
+                step = std::max(step, iterations_ahead(J, P.host_st[i].residual, P.host_st[i].iter, tol));
     }
     for (int i = 0; i < N; ++i) {
         const auto& g = P.views[i].mem;
