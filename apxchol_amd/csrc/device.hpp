@@ -78,7 +78,10 @@ struct pcg_state {
     double out_sum;      // sum of the last application's output
     double mu;           // output-centring shift of the last application
     double beta;
-    double pad[4];
+    // r.z of a single-vector solve by the parity of the iteration: the kernel
+    // that forms the new one (in every workgroup) still reads the old one.
+    double rz_by_parity[2];
+    double pad[2];
     int iter, done, max_iter, stag_window;
     int apply_count, center_k, laplacian, center_now;
     int status;          // 0 running, 1 converged, 2 breakdown (pAp <= 0), 3 stagnation, 4 max_iter,
@@ -87,6 +90,15 @@ struct pcg_state {
     int phase;           // blocked solves: 0 iterating, 1 joining (first application pending)
     int pad_i;
 };
+
+// A reduction of at most this many partials is finished by its consumer, every
+// workgroup for itself, instead of a launch of its own (see update_xr_body);
+// update_xr's own partials then start at kFusedPartOffset, past those it reads.
+// fp64 solves of 3-D SDDM grids, always against never: 40^3 2,265 / 2,348 us,
+// 50^3 2,916 / 2,989, 57^3 3,888 / 3,978, 64^3 (1024 partials) 4,720 / 4,782,
+// 72^3 within the noise, 80^3 (2000) 8,099 / 8,001.
+inline constexpr int kFuseBlocks = 1024;
+inline constexpr int kFusedPartOffset = 8192;
 
 // Partials a column of a blocked reduction may have: the vector kernels' grid
 // cap (2048), the SpMM's rounding up and the long rows' one more.

@@ -872,7 +872,8 @@ void gpu_solver::setup(const csc_view& L) {
     const std::size_t vb = static_cast<std::size_t>(std::max(n, 1)) * sizeof(double);
     d.r.alloc(vb); d.x.alloc(vb); d.p.alloc(vb); d.ap.alloc(vb); d.rp.alloc(vb); d.y.alloc(vb); d.z.alloc(vb);
     d.xout.alloc(vb);
-    d.part.alloc(2 * static_cast<std::size_t>(std::max(kMaxBlocksHost, kSellMaxBlocks)) * sizeof(double));
+    static_assert(kSellMaxBlocks <= kFusedPartOffset && 2 * kMaxBlocksHost <= kFusedPartOffset, "partials");
+    d.part.alloc(2 * static_cast<std::size_t>(kFusedPartOffset) * sizeof(double));
     d.st.alloc(sizeof(pcg_state));
     d.st_apply.alloc(sizeof(pcg_state));
     d.st_apply.zero();
@@ -1377,19 +1378,20 @@ void gpu_solver::enqueue_precondition(bool first, int step, hipStream_t s) const
     if (first) launch_fill_outputs(pr, n, m, sentinel_y, d.z.get(), st, s);
     enqueue_pair(d.r.as<double>(), st, step, s);
     tm.time(3, step, s, [&] {
-        launch_dot_center(pr, n, d.r.as<double>(), d.z.get(), st, part, first, s);
-        launch_update_p(pr, n, d.p.as<double>(), d.z.get(), st, first, s);
+        int deferred = 0;
+        launch_dot_center(pr, n, d.r.as<double>(), d.z.get(), st, part, first, s, &deferred);
+        launch_update_p(pr, n, d.p.as<double>(), d.z.get(), st, part, first, deferred, s);
     });
 }
 
 void gpu_solver::spmv(const double* x, double* y, pcg_state* st, bool want_dot, hipStream_t s,
-                      const launch_hook& hook) const {
+                      const launch_hook& hook, int* defer) const {
     auto& d = *dev_;
     if (d.use_sell)
-        launch_spmv_sell(d.sell, d.op32, x, y, st, d.part.as<double>(), want_dot, s, hook);
+        launch_spmv_sell(d.sell, d.op32, x, y, st, d.part.as<double>(), want_dot, s, hook, defer);
     else
         launch_spmv(static_cast<int>(n_), d.op_ptr.as<unsigned>(), d.op_idx.as<int>(), d.op_val.get(), d.op32, d.lanes,
-                    x, y, st, d.part.as<double>(), want_dot, s, hook);
+                    x, y, st, d.part.as<double>(), want_dot, s, hook, defer);
 }
 
 void gpu_solver::enqueue_iteration(int it, hipStream_t s) const {
@@ -1399,10 +1401,12 @@ void gpu_solver::enqueue_iteration(int it, hipStream_t s) const {
     const int m = static_cast<int>(T_.m);
     pcg_state* st = d.st.as<pcg_state>();
     double* part = d.part.as<double>();
-    spmv(d.p.as<double>(), d.ap.as<double>(), st, true, s, tm.hook(it - 1));
+    int deferred = 0;
+    spmv(d.p.as<double>(), d.ap.as<double>(), st, true, s, tm.hook(it - 1), &deferred);
     tm.time(3, it - 1, s, [&] {
         launch_update_xr(d.prec, n, m, d.x.as<double>(), d.p.as<double>(), d.r.as<double>(), d.ap.as<double>(),
-                         opts_.schedule == sweep_schedule::dataflow ? d.y.get() : nullptr, d.z.get(), st, part, s);
+                         opts_.schedule == sweep_schedule::dataflow ? d.y.get() : nullptr, d.z.get(), st, part,
+                         deferred, s);
     });
     enqueue_precondition(false, it, s);
 }

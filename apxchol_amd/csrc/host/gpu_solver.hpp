@@ -266,7 +266,8 @@ private:
     // preconditioned dot and the p update); step labels the timing records.
     void enqueue_iteration(int step, hipStream_t s) const;
     // y = A x with the solver's single-vector SpMV (sliced ELL or CSR lanes).
-    void spmv(const double* x, double* y, pcg_state* st, bool want_dot, hipStream_t s, const launch_hook& hook) const;
+    void spmv(const double* x, double* y, pcg_state* st, bool want_dot, hipStream_t s, const launch_hook& hook,
+              int* defer = nullptr) const;
     void enqueue_precondition(bool first, int step, hipStream_t s) const;
     // Forms the trailing block of the rows from `first` on; false (and no
     // block) when its inverse leaves the vectors' range.

@@ -64,6 +64,9 @@ struct solver_group::impl {
     pcg_state* host_st = nullptr;
     devmem starts;               // every starts array, back to back
     int spmv_s = 0, spmv_blocks = 0, vec_s = 0, vec_blocks = 0;
+    // Stage 2 of the reductions left to their consumers (every member's
+    // partials few enough).
+    bool fuse_pAp = false, fuse_dot = false;
     // One sweep step: its level units, then its tail units, in units[dir].
     struct step {
         int lv_off = 0, lv_count = 0, lv_s = 0, lv_blocks = 0;
@@ -107,15 +110,15 @@ struct solver_group::impl {
                            tr_couple_blocks, tr_apply_blocks, tr_lds, s);
         sweep(1, s);
         launch_group_dot_center(prec, M(), S(vec_s), count, vec_blocks, s);
-        launch_group_finish(group_fin_op(first ? "dot_first" : "dot"), M(), S(vec_s), count, s);
-        launch_group_update_p(prec, M(), S(vec_s), count, vec_blocks, first, s);
+        if (!fuse_dot) launch_group_finish(group_fin_op(first ? "dot_first" : "dot"), M(), S(vec_s), count, 0, s);
+        launch_group_update_p(prec, M(), S(vec_s), count, vec_blocks, first, fuse_dot, s);
     }
     // One PCG iteration of every member (gpu_solver::enqueue_iteration).
     void iteration(hipStream_t s) const {
         launch_group_spmv(M(), S(spmv_s), count, spmv_blocks, s);
-        launch_group_finish(group_fin_op("pAp"), M(), S(spmv_s), count, s);
-        launch_group_update_xr(prec, M(), S(vec_s), count, vec_blocks, s);
-        launch_group_finish(group_fin_op("xr"), M(), S(vec_s), count, s);
+        if (!fuse_pAp) launch_group_finish(group_fin_op("pAp"), M(), S(spmv_s), count, 0, s);
+        launch_group_update_xr(prec, M(), S(vec_s), count, vec_blocks, fuse_pAp ? S(spmv_s) : nullptr, s);
+        launch_group_finish(group_fin_op("xr"), M(), S(vec_s), count, fuse_pAp ? kFusedPartOffset : 0, s);
         precondition(false, s);
     }
 };
@@ -163,7 +166,10 @@ solver_group::solver_group(std::vector<std::shared_ptr<const gpu_solver>> member
     };
     P.spmv_s = add(g_spmv, P.spmv_blocks);
     P.vec_s = add(g_vec, P.vec_blocks);
-    int launches = 4 + 3;   // spmv, finish, update_xr, finish; dot_center, finish, update_p
+    P.fuse_pAp = *std::max_element(g_spmv.begin(), g_spmv.end()) <= kFuseBlocks;
+    P.fuse_dot = *std::max_element(g_vec.begin(), g_vec.end()) <= kFuseBlocks;
+    // spmv, finish, update_xr, finish; dot_center, finish, update_p
+    int launches = 4 + 3 - (P.fuse_pAp ? 1 : 0) - (P.fuse_dot ? 1 : 0);
     // Sweep steps, aligned at each member's last step.
     for (int dir = 0; dir < 2; ++dir) {
         std::size_t S = 0;

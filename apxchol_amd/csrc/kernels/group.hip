@@ -63,20 +63,24 @@ __global__ __launch_bounds__(kBlock) void group_spmv(const group_member* __restr
 // Stage 2 of a reduction for every member (workgroup i: member i; its
 // producer's grid is starts[i + 1] - starts[i]).
 __global__ __launch_bounds__(kBlock) void group_finish(int op, const group_member* __restrict__ mem,
-                                                       const int* __restrict__ starts) {
+                                                       const int* __restrict__ starts, int offset) {
     const int i = static_cast<int>(blockIdx.x);
     const group_member& g = mem[i];
-    pcg_finish_body(op, g.n, g.part, starts[i + 1] - starts[i], g.st);
+    pcg_finish_body(op, g.n, g.part + offset, starts[i + 1] - starts[i], g.st);
 }
 
 template <class TO>
 __global__ __launch_bounds__(kBlock) void group_update_xr(const group_member* __restrict__ mem,
-                                                          const int* __restrict__ starts, int count) {
+                                                          const int* __restrict__ starts, int count,
+                                                          const int* __restrict__ dot_starts) {
     const int b = static_cast<int>(blockIdx.x);
     const int i = group_unit_of(starts, count, b);
     const group_member& g = mem[i];
+    // dot_starts: the SpMV's grids when its partials are summed here.
     update_xr_body<TO>(b - starts[i], starts[i + 1] - starts[i], g.n, g.m, g.x, g.p, g.r, g.ap,
-                       static_cast<TO*>(nullptr), static_cast<TO*>(g.z), g.st, g.part);
+                       static_cast<TO*>(nullptr), static_cast<TO*>(g.z), g.st,
+                       g.part + (dot_starts ? kFusedPartOffset : 0), g.part,
+                       dot_starts ? dot_starts[i + 1] - dot_starts[i] : 0);
 }
 
 template <class TO>
@@ -101,11 +105,13 @@ __global__ __launch_bounds__(kBlock) void group_dot_center(const group_member* _
 
 template <class TO>
 __global__ __launch_bounds__(kBlock) void group_update_p(const group_member* __restrict__ mem,
-                                                         const int* __restrict__ starts, int count, int first) {
+                                                         const int* __restrict__ starts, int count, int first,
+                                                         int fused) {
     const int b = static_cast<int>(blockIdx.x);
     const int i = group_unit_of(starts, count, b);
     const group_member& g = mem[i];
-    update_p_body<TO>(b - starts[i], starts[i + 1] - starts[i], g.n, g.p, static_cast<const TO*>(g.z), g.st, first);
+    const int vg = starts[i + 1] - starts[i];
+    update_p_body<TO>(b - starts[i], vg, g.n, g.p, static_cast<const TO*>(g.z), g.st, first, g.part, fused ? vg : 0);
 }
 
 // One step of the members' sweeps: launched levels from the lane layout or

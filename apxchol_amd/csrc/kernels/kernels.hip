@@ -260,9 +260,19 @@ void finish(int op, int n, const double* part, int nb, pcg_state* st, hipStream_
     check_launch("pcg_finish");
 }
 
+// Stage 2 of a reduction some launches support summing in its consumer (defer
+// given): with few enough partials their number goes to *defer instead (else 0).
+static void finish_or_defer(bool want, int op, int n, const double* part, int nb, pcg_state* st, hipStream_t s,
+                            int* defer) {
+    if (defer) *defer = 0;
+    if (!want) return;
+    if (defer && nb <= kFuseBlocks) *defer = nb;
+    else finish(op, n, part, nb, st, s);
+}
+
 template <class VT>
 static void spmv_t(int n, const unsigned* ptr, const int* idx, const VT* val, int lanes, const double* x, double* y,
-                   pcg_state* st, double* part, bool want_dot, hipStream_t s, const launch_hook& hook) {
+                   pcg_state* st, double* part, bool want_dot, hipStream_t s, const launch_hook& hook, int* defer) {
     const int g = vec_blocks(static_cast<long long>(n) * lanes);
     const int w = want_dot ? 1 : 0;
     auto go = [&](auto kernel) {
@@ -278,18 +288,20 @@ static void spmv_t(int n, const unsigned* ptr, const int* idx, const VT* val, in
         default: go(spmv_pAp<VT, 64>); break;
     }
     check_launch("spmv_pAp");
-    if (want_dot) finish(kFinPAp, n, part, g, st, s);
+    finish_or_defer(want_dot, kFinPAp, n, part, g, st, s, defer);
 }
 
 void launch_spmv(int n, const unsigned* ptr, const int* idx, const void* val, bool val32, int lanes, const double* x,
-                 double* y, pcg_state* st, double* part, bool want_dot, hipStream_t s, const launch_hook& hook) {
+                 double* y, pcg_state* st, double* part, bool want_dot, hipStream_t s, const launch_hook& hook,
+                 int* defer) {
     if (want_dot && !st) throw std::invalid_argument("apxchol_amd: SpMV dot product without a solve state");
-    if (val32) spmv_t<float>(n, ptr, idx, static_cast<const float*>(val), lanes, x, y, st, part, want_dot, s, hook);
-    else spmv_t<double>(n, ptr, idx, static_cast<const double*>(val), lanes, x, y, st, part, want_dot, s, hook);
+    if (val32) spmv_t<float>(n, ptr, idx, static_cast<const float*>(val), lanes, x, y, st, part, want_dot, s, hook, defer);
+    else spmv_t<double>(n, ptr, idx, static_cast<const double*>(val), lanes, x, y, st, part, want_dot, s, hook, defer);
 }
 
 void launch_spmv_sell(const sell_desc& a, bool val32, const double* x, double* y, pcg_state* st, double* part,
-                      bool want_dot, hipStream_t s, const launch_hook& hook) {
+                      bool want_dot, hipStream_t s, const launch_hook& hook, int* defer) {
+    if (defer) *defer = 0;
     if (want_dot && !st) throw std::invalid_argument("apxchol_amd: SpMV dot product without a solve state");
     const long long items = static_cast<long long>(a.nslices) + a.nlong;
     if (items <= 0) return;
@@ -309,7 +321,7 @@ void launch_spmv_sell(const sell_desc& a, bool val32, const double* x, double* y
         else go(spmv_sell<double, false>);
     }
     check_launch("spmv_sell");
-    if (want_dot) finish(kFinPAp, a.n, part, static_cast<int>(g), st, s);
+    finish_or_defer(want_dot, kFinPAp, a.n, part, static_cast<int>(g), st, s, defer);
 }
 
 void launch_scatter_init(int n, const unsigned* perm, const double* b, const double* x0, double* r, double* x,
@@ -333,29 +345,35 @@ void launch_init_residual(int n, double* r, const double* ax0, pcg_state* st, do
 }
 
 void launch_update_xr(vec_prec p, int n, int m, double* x, const double* pv, double* r, const double* ap, void* y,
-                      void* z, pcg_state* st, double* part, hipStream_t s) {
+                      void* z, pcg_state* st, double* part, int deferred, hipStream_t s) {
     const int g = vec_blocks(n);
+    double* own = part + (deferred > 0 ? kFusedPartOffset : 0);
     if (p == vec_prec::fp64)
-        update_xr<double><<<g, kBlock, 0, s>>>(n, m, x, pv, r, ap, static_cast<double*>(y), static_cast<double*>(z), st, part);
+        update_xr<double><<<g, kBlock, 0, s>>>(n, m, x, pv, r, ap, static_cast<double*>(y), static_cast<double*>(z), st,
+                                               own, part, deferred);
     else
-        update_xr<float><<<g, kBlock, 0, s>>>(n, m, x, pv, r, ap, static_cast<float*>(y), static_cast<float*>(z), st, part);
+        update_xr<float><<<g, kBlock, 0, s>>>(n, m, x, pv, r, ap, static_cast<float*>(y), static_cast<float*>(z), st,
+                                              own, part, deferred);
     check_launch("update_xr");
-    finish(kFinXR, n, part, g, st, s);
+    finish(kFinXR, n, own, g, st, s);
 }
 
 void launch_dot_center(vec_prec p, int n, const double* r, const void* out, pcg_state* st, double* part, bool first,
-                       hipStream_t s) {
+                       hipStream_t s, int* defer) {
     const int g = vec_blocks(n);
     if (p == vec_prec::fp64) dot_center<double><<<g, kBlock, 0, s>>>(n, r, static_cast<const double*>(out), st, part);
     else dot_center<float><<<g, kBlock, 0, s>>>(n, r, static_cast<const float*>(out), st, part);
     check_launch("dot_center");
-    finish(first ? kFinDotFirst : kFinDot, n, part, g, st, s);
+    finish_or_defer(true, first ? kFinDotFirst : kFinDot, n, part, g, st, s, defer);
 }
 
-void launch_update_p(vec_prec p, int n, double* pv, const void* out, const pcg_state* st, bool first, hipStream_t s) {
+void launch_update_p(vec_prec p, int n, double* pv, const void* out, pcg_state* st, const double* part, bool first,
+                     int deferred, hipStream_t s) {
     const int g = vec_blocks(n);
-    if (p == vec_prec::fp64) update_p<double><<<g, kBlock, 0, s>>>(n, pv, static_cast<const double*>(out), st, first ? 1 : 0);
-    else update_p<float><<<g, kBlock, 0, s>>>(n, pv, static_cast<const float*>(out), st, first ? 1 : 0);
+    if (p == vec_prec::fp64)
+        update_p<double><<<g, kBlock, 0, s>>>(n, pv, static_cast<const double*>(out), st, first ? 1 : 0, part, deferred);
+    else
+        update_p<float><<<g, kBlock, 0, s>>>(n, pv, static_cast<const float*>(out), st, first ? 1 : 0, part, deferred);
     check_launch("update_p");
 }
 
@@ -1004,17 +1022,17 @@ void launch_group_spmv(const group_member* mem, const int* starts, int count, in
     check_launch("group_spmv");
 }
 
-void launch_group_finish(int op, const group_member* mem, const int* starts, int count, hipStream_t s) {
+void launch_group_finish(int op, const group_member* mem, const int* starts, int count, int offset, hipStream_t s) {
     if (count <= 0) return;
-    group_finish<<<count, kBlock, 0, s>>>(op, mem, starts);
+    group_finish<<<count, kBlock, 0, s>>>(op, mem, starts, offset);
     check_launch("group_finish");
 }
 
 void launch_group_update_xr(vec_prec p, const group_member* mem, const int* starts, int count, int blocks,
-                            hipStream_t s) {
+                            const int* dot_starts, hipStream_t s) {
     if (count <= 0 || blocks <= 0) return;
-    if (p == vec_prec::fp64) group_update_xr<double><<<blocks, kBlock, 0, s>>>(mem, starts, count);
-    else group_update_xr<float><<<blocks, kBlock, 0, s>>>(mem, starts, count);
+    if (p == vec_prec::fp64) group_update_xr<double><<<blocks, kBlock, 0, s>>>(mem, starts, count, dot_starts);
+    else group_update_xr<float><<<blocks, kBlock, 0, s>>>(mem, starts, count, dot_starts);
     check_launch("group_update_xr");
 }
 
@@ -1035,10 +1053,10 @@ void launch_group_dot_center(vec_prec p, const group_member* mem, const int* sta
 }
 
 void launch_group_update_p(vec_prec p, const group_member* mem, const int* starts, int count, int blocks, bool first,
-                           hipStream_t s) {
+                           bool fused, hipStream_t s) {
     if (count <= 0 || blocks <= 0) return;
-    if (p == vec_prec::fp64) group_update_p<double><<<blocks, kBlock, 0, s>>>(mem, starts, count, first ? 1 : 0);
-    else group_update_p<float><<<blocks, kBlock, 0, s>>>(mem, starts, count, first ? 1 : 0);
+    if (p == vec_prec::fp64) group_update_p<double><<<blocks, kBlock, 0, s>>>(mem, starts, count, first ? 1 : 0, fused ? 1 : 0);
+    else group_update_p<float><<<blocks, kBlock, 0, s>>>(mem, starts, count, first ? 1 : 0, fused ? 1 : 0);
     check_launch("group_update_p");
 }
 

@@ -122,21 +122,27 @@ void launch_fill_outputs(vec_prec p, int n, int m, void* y, void* z, const pcg_s
 
 void launch_spmv(int n, const unsigned* ptr, const int* idx, const void* val, bool val32, int lanes, const double* x,
                  double* y, pcg_state* st, double* part, bool want_dot, hipStream_t s,
-                 const launch_hook& hook = {});
+                 const launch_hook& hook = {}, int* defer = nullptr);
 
 // y = A x (and x.y into st->pAp when want_dot) over the sliced-ELL form.
 void launch_spmv_sell(const sell_desc& a, bool val32, const double* x, double* y, pcg_state* st, double* part,
-                      bool want_dot, hipStream_t s, const launch_hook& hook = {});
+                      bool want_dot, hipStream_t s, const launch_hook& hook = {}, int* defer = nullptr);
 
 void launch_scatter_init(int n, const unsigned* perm, const double* b, const double* x0, double* r, double* x,
                          hipStream_t s);
 void launch_norm2_b(int n, const double* b, pcg_state* st, double* part, hipStream_t s);
 void launch_init_residual(int n, double* r, const double* ax0, pcg_state* st, double* part, hipStream_t s);
-// x, r update and its reductions; y, z as in launch_fill_outputs (y null: no sentinels).
+// x, r update and its reductions; y, z as in launch_fill_outputs (y null: no
+// sentinels). A launch given `defer` may leave stage 2 of its reduction to the
+// next one: *defer is then the number of its partials (else 0), which the
+// consumer takes as `deferred` (update_xr those of the SpMV, update_p those of
+// dot_center).
 void launch_update_xr(vec_prec p, int n, int m, double* x, const double* pv, double* r, const double* ap, void* y,
-                      void* z, pcg_state* st, double* part, hipStream_t s);
-void launch_dot_center(vec_prec p, int n, const double* r, const void* out, pcg_state* st, double* part, bool first, hipStream_t s);
-void launch_update_p(vec_prec p, int n, double* pv, const void* out, const pcg_state* st, bool first, hipStream_t s);
+                      void* z, pcg_state* st, double* part, int deferred, hipStream_t s);
+void launch_dot_center(vec_prec p, int n, const double* r, const void* out, pcg_state* st, double* part, bool first,
+                       hipStream_t s, int* defer = nullptr);
+void launch_update_p(vec_prec p, int n, double* pv, const void* out, pcg_state* st, const double* part, bool first,
+                     int deferred, hipStream_t s);
 void launch_sum_vec(int n, const double* a, pcg_state* st, double* part, hipStream_t s);
 void launch_gather_shift(int n, const unsigned* perm, const double* src, double* dst, const pcg_state* st,
                          bool use_mean, hipStream_t s);
@@ -283,15 +289,19 @@ struct group_unit {
 int group_spmv_blocks(const group_member& g);
 int group_vec_blocks(int n);
 void launch_group_spmv(const group_member* mem, const int* starts, int count, int blocks, hipStream_t s);
-void launch_group_finish(int op, const group_member* mem, const int* starts, int count, hipStream_t s);
+// offset: where the members' partials start in their buffers.
+void launch_group_finish(int op, const group_member* mem, const int* starts, int count, int offset, hipStream_t s);
+// dot_starts: the SpMV's starts when stage 2 of its reduction is left to this
+// launch (its own partials then lie at kFusedPartOffset); else null.
 void launch_group_update_xr(vec_prec p, const group_member* mem, const int* starts, int count, int blocks,
-                            hipStream_t s);
+                            const int* dot_starts, hipStream_t s);
 void launch_group_fill_outputs(vec_prec p, const group_member* mem, const int* starts, int count, int blocks,
                                hipStream_t s);
 void launch_group_dot_center(vec_prec p, const group_member* mem, const int* starts, int count, int blocks,
                              hipStream_t s);
+// fused: stage 2 of dot_center's reduction is left to this launch.
 void launch_group_update_p(vec_prec p, const group_member* mem, const int* starts, int count, int blocks, bool first,
-                           hipStream_t s);
+                           bool fused, hipStream_t s);
 // One step of the members' sweeps in one direction: the launched levels, the
 // coupling launches of the tail runs, then the tail runs (count units each).
 void launch_group_sweep_level(vec_prec p, bool fp16, bool backward, const group_unit* units, const int* starts,
