@@ -177,6 +177,22 @@ struct alignas(8) lane_rec {
     std::uint32_t info;  // log2 G | sub << 3 | nvalid << 9
 };
 
+// Level tiles (kernels/tile.hip): `levels` consecutive levels from `level` on in
+// one launch of `tiles` workgroups. Tile k's batches of level p are the
+// width[p] lane batches from base[p] + k * width[p] on. lane_rec::info also
+// holds the row's slot in the tile's outputs (from bit kTileSlotShift on) and
+// whether the tile writes it out (kTileOwn); ent.idx < 0: slot ~idx of the
+// tile's outputs instead of a row.
+inline constexpr int kTileMaxLevels = 4;
+inline constexpr int kTileWaves = 16;
+inline constexpr int kTileSlotShift = 12;
+inline constexpr std::uint32_t kTileOwn = 1u << 28;
+static_assert(kTileMaxLevels * kTileWaves * kWave <= 1 << 16, "slots of a tile");
+struct tile_step {
+    int level = 0, levels = 0, tiles = 0, slots = 0;
+    int base[kTileMaxLevels] = {}, width[kTileMaxLevels] = {};
+};
+
 // The trailing block: the last n rows of the factor (storage rows [first,
 // first + n)), applied through its explicit inverse S = T^-T W T^-1 (see
 // kernels/trail.hip). The coupling to the rows before it comes as lane batches

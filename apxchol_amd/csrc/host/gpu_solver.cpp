@@ -23,6 +23,7 @@
 #include "../device.hpp"
 #include "../kernels/launch.hpp"
 #include "merge.hpp"
+#include "tile.hpp"
 #include "trail.hpp"
 
 namespace apxchol_amd {
@@ -506,6 +507,8 @@ struct gpu_solver::device_state {
     std::vector<int> f_levels, b_levels;
     dbuf f_levels_dev, b_levels_dev, tail_val;
     dbuf f_tlane, f_tent, f_tovf, f_tovf_ent, f_twalk, b_tlane, b_tent, b_tovf, b_tovf_ent, b_twalk;
+    std::vector<tile_step> tiles[2];   // level tiles of the forward and the back sweep
+    dbuf tile_rec[2], tile_ent[2];
     dbuf f_tlane_r, b_tlane_r;   // tail lanes with 1 / diag (fp32-vector sweeps)
     dbuf f_lrec, f_lent, b_lrec, b_lent;
     std::vector<int> f_level_lb, b_level_lb;   // first lane batch of each level, or -1
@@ -952,6 +955,14 @@ void gpu_solver::setup(const csc_view& L) {
     if (const char* e = std::getenv("APXCHOL_AMD_TRAIL_ROWS"); e && *e) trail_max = std::max(0, std::atoi(e));
     std::size_t cut = choose_trail_level(T_, d.prec == vec_prec::fp64 ? 8 : 4, d.f_levels, d.b_levels, trail_max);
     if (cut < L_all && !build_trail(T_.level_ptr[cut])) cut = L_all;
+    // What the level tiles of a direction are built from.
+    struct tile_input {
+        lane_tables lt;
+        std::vector<int> level_pos;
+        std::vector<std::pair<int, int>> runs;
+        tile_tables out;
+    };
+    tile_input tile_in[2];
     auto make_sched = [&](sweep_sched& sc, const batch_table& bt, bool backward, const std::vector<int>& lf,
                           dbuf& lf_dev, std::vector<int> (&seg)[8], dbuf* const (&tbuf)[6], std::vector<int>& level_lb,
                           dbuf& lrec, dbuf& lent, std::vector<int>& level_pos, std::vector<unsigned char>& level_diag) {
@@ -1106,6 +1117,24 @@ void gpu_solver::setup(const csc_view& L) {
         sc.lane_rec_dev = lrec.as<lane_rec>();
         sc.lane_ent_dev = lent.as<entry32>();
         sc.lane_batches = lt.batches;
+        // Runs of launched levels of at most tile_batches batches may be joined
+        // in tiles, none across the trailing block's boundary. A level of more
+        // batches is bound by its bytes: joining those too (4,096) gains
+        // nothing on a mixed 128^3 solve and doubles the host's time.
+        const int tile_batches = env_int("APXCHOL_AMD_TILE_BATCHES", 2048);
+        tile_input& ti = tile_in[backward ? 1 : 0];
+        if (sc.kind == 2) {
+            for (int q = 0; q <= L; ++q) ti.level_pos.push_back(pos(q));
+            const auto fits = [&](int q) { return level_lb[q] >= 0 && lf[q + 1] - lf[q] <= tile_batches; };
+            for (int l = 0; l < L;) {
+                if (!fits(l)) { ++l; continue; }
+                int e = l + 1;
+                while (e < L && e != cl && fits(e)) ++e;
+                ti.runs.emplace_back(l, e);
+                l = e;
+            }
+        }
+        ti.lt = std::move(lt);
         // Big launched levels run several batches per wave (fewer waves to
         // dispatch; the same bits).
         sc.lane_bpw2 = env_int("APXCHOL_AMD_LANE_BPW2", 0);
@@ -1181,12 +1210,60 @@ void gpu_solver::setup(const csc_view& L) {
                d.f_level_pos, d.f_level_diag);
     make_sched(d.b_sched, bb, true, d.b_levels, d.b_levels_dev, d.b_seg, b_tb, d.b_level_lb, d.b_lrec, d.b_lent,
                d.b_level_pos, d.b_level_diag);
+    long long growth = opts_.merge_levels ? -1 : 0;
+    if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
+    const bool merging = d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0;
+    // Level tiles, the two directions side by side, where levels are not merged
+    // (APXCHOL_AMD_TILE_LEVELS: levels a launch may join, 1: none). A solver for
+    // one solve goes without: on a mixed 128^3 system they take 0.2 s and save
+    // 2.3 ms a solve.
+    const int tile_levels = env_int("APXCHOL_AMD_TILE_LEVELS", opts_.merge_levels ? kTileMaxLevels : 1);
+    if (tile_levels > 1 && !merging) {
+        const auto build = [&](int dir) {
+            tile_input& t = tile_in[dir];
+            for (const auto& run : t.runs)
+                append_tiles(t.lt, dir != 0, static_cast<std::uint32_t>(m), dir ? d.b_levels : d.f_levels,
+                             dir ? d.b_level_lb : d.f_level_lb, t.level_pos, run.first, run.second, tile_levels, t.out);
+        };
+        std::exception_ptr failed;
+        std::thread back([&] {
+            try {
+                build(1);
+            } catch (...) {
+                failed = std::current_exception();
+            }
+        });
+        try {
+            build(0);
+        } catch (...) {
+            back.join();
+            throw;
+        }
+        back.join();
+        if (failed) std::rethrow_exception(failed);
+        for (int dir = 0; dir < 2; ++dir) {
+            sweep_sched& sc = dir ? d.b_sched : d.f_sched;
+            tile_tables& t = tile_in[dir].out;
+            d.tiles[dir] = std::move(t.steps);
+            if (d.tiles[dir].empty()) continue;
+            d.tile_rec[dir].upload(t.rec);
+            d.tile_ent[dir].upload(t.ent);
+            sc.tiles = d.tiles[dir].data();
+            sc.ntiles = static_cast<int>(d.tiles[dir].size());
+            sc.tile_rec_dev = d.tile_rec[dir].as<lane_rec>();
+            sc.tile_ent_dev = d.tile_ent[dir].as<entry32>();
+            sc.tile_batches = t.batches;
+            for (const tile_step& x : d.tiles[dir]) {
+                stats_.level_launches[dir] -= x.levels - 1;
+                if (cut == L_all || (dir ? x.level >= sc.cut_level : x.level < sc.cut_level))
+                    stats_.solve_level_launches[dir] -= x.levels - 1;
+            }
+        }
+    }
     // An application's steps outside the trailing block, the two directions side
     // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
     // may gain; 0: no merging).
-    long long growth = opts_.merge_levels ? -1 : 0;
-    if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
-    if (d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0) {
+    if (merging) {
         const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
         merge_tables mt[2];
         std::exception_ptr failed;

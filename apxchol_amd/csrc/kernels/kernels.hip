@@ -15,6 +15,7 @@
 #include "block.hip"
 #include "trail.hip"
 #include "merge.hip"
+#include "tile.hip"
 #include "pieces.hip"
 #include "group.hip"
 
@@ -169,8 +170,29 @@ void sweep_t(const sweep_desc& d, const void* rhs, void* out, const pcg_state* s
             launch_timed(hook, 2, sweep_couple<TI, TO, F16, kWave>, dim3(bl - bf), dim3(kWave), 0, on, d, bf, bl, plo,
                          phi, cont, in, static_cast<const TO*>(o), tv, st, 1, static_cast<const batch_state*>(nullptr));
         };
+        // Step of level tiles that starts at level l, if any.
+        int ti = 0;
+        const auto tile_at = [&](int l) -> const tile_step* {
+            while (ti < sc.ntiles && sc.tiles[ti].level < l) ++ti;
+            return ti < sc.ntiles && sc.tiles[ti].level == l ? &sc.tiles[ti] : nullptr;
+        };
         for (int k = k0; k < k1; ++k) {
             if (!sc.seg_tail[k]) {
+                if (const tile_step* t = tile_at(sc.seg_l0[k])) {
+                    for (int p = 0; p < t->levels; ++p)
+                        if (k + p >= k1 || sc.seg_tail[k + p] || sc.seg_l0[k + p] != t->level + p ||
+                            t->base[p] + static_cast<long long>(t->tiles) * t->width[p] > sc.tile_batches)
+                            throw std::runtime_error("apxchol_amd: level tiles outside their layout");
+                    const int waves = *std::max_element(t->width, t->width + t->levels);
+                    const auto f = t->levels == 2   ? sweep_tiles<TI, TO, 2>
+                                   : t->levels == 3 ? sweep_tiles<TI, TO, 3>
+                                                    : sweep_tiles<TI, TO, 4>;
+                    launch_timed(hook, 0, f, dim3(t->tiles), dim3(waves * kWave),
+                                 static_cast<unsigned>(t->slots * sizeof(TO)), s, d, *t, sc.tile_rec_dev,
+                                 sc.tile_ent_dev, in, o, st);
+                    k += t->levels - 1;
+                    continue;
+                }
                 for (int l = sc.seg_l0[k]; l < sc.seg_l1[k]; ++l) level_launch(l);
                 continue;
             }

@@ -64,6 +64,13 @@ struct sweep_sched {
     long long lane_batches = 0;
     int lane_bpw2 = 0;                     // lane levels of >= this many batches: 2 per wave (0: never)
     int lane_bpw4 = 0;                     // ... >= this many: 4 per wave (0: never)
+    // Launched levels joined in level tiles (host; ascending, none across the
+    // trailing block's boundary).
+    const tile_step* tiles = nullptr;
+    int ntiles = 0;
+    const lane_rec* tile_rec_dev = nullptr;
+    const entry32* tile_ent_dev = nullptr;
+    long long tile_batches = 0;
     // The boundary of the trailing block in this direction: its first level,
     // segment and batch (back sweep: the first ones after it).
     int cut_level = 0, cut_seg = 0, cut_batch = 0;
