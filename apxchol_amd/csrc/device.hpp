@@ -55,10 +55,18 @@ struct sweep_desc {
 //                                      (padding: the row itself / 0, value 0)
 // Rows too long for a slice are listed in longrows and read from the CSR
 // arrays (ptr, cidx, cval) by a whole wave.
+// A long row of more entries than 1/1024 of all in long rows, at least
+// kHugeRowMin and at most kHugeRowMax, is summed a wave per column by the SpMM,
+// a shorter one by one wave for all columns (spmm_long_k), which is cheaper
+// unless the launch ends up waiting for it. 32 columns, R-MAT scale 14 / 18, ms:
+// above 1024 0.13 / 1.38, above 4096 0.27 / 0.93, every row a wave per column
+// (entries past 8 times the mean only; the others in slices) 0.16 / 1.42.
+inline constexpr int kHugeRowMin = 1024, kHugeRowMax = 4096;
 struct sell_desc {
     int n = 0;
     int nslices = 0;
     int nlong = 0;
+    int nhuge = 0;                          // huge ones among the long rows (the first: longest first)
     int max_blocks = 2048;                  // workgroup cap of the launch (partials buffer size)
     const std::uint32_t* soff = nullptr;
     const std::int32_t* idx = nullptr;
@@ -101,8 +109,9 @@ inline constexpr int kFuseBlocks = 1024;
 inline constexpr int kFusedPartOffset = 8192;
 
 // Partials a column of a blocked reduction may have: the vector kernels' grid
-// cap (2048), the SpMM's rounding up and the long rows' one more.
-inline constexpr int kColPartials = 2080;
+// cap (2048), the SpMM's rounding up and the long rows' own.
+inline constexpr int kColPartials = 2304;
+inline constexpr int kLongDotBlocks = 224;   // workgroups of spmm_long_dot_k
 
 // Bookkeeping of a blocked (k right-hand sides) solve: the number of columns
 // still iterating; every blocked kernel returns at once when it is zero.

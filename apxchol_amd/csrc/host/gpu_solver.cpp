@@ -858,6 +858,13 @@ void gpu_solver::setup(const csc_view& L) {
                     d.sell.max_blocks = std::clamp(std::atoi(gb), kXcdsHost, kSellMaxBlocks);
                 d.sell.nslices = static_cast<int>(sl.soff.size()) - 1;
                 d.sell.nlong = static_cast<int>(sl.longrows.size());
+                std::uint64_t in_long = 0;
+                for (const std::int32_t r : sl.longrows) in_long += op.ptr[r + 1] - op.ptr[r];
+                const std::uint32_t huge = static_cast<std::uint32_t>(
+                    std::clamp<std::uint64_t>(in_long / 1024, kHugeRowMin, kHugeRowMax));
+                d.sell.nhuge = static_cast<int>(std::partition_point(sl.longrows.begin(), sl.longrows.end(), [&](std::int32_t r) {
+                    return op.ptr[r + 1] - op.ptr[r] > huge;
+                }) - sl.longrows.begin());
                 d.sell.soff = d.sell_soff.as<std::uint32_t>();
                 d.sell.idx = d.sell_idx.as<std::int32_t>();
                 d.sell.val = d.sell_val.get();
@@ -1212,7 +1219,36 @@ void gpu_solver::setup(const csc_view& L) {
                d.b_level_pos, d.b_level_diag);
     long long growth = opts_.merge_levels ? -1 : 0;
     if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
-    const bool merging = d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0;
+    // (Of 1024 levels and more outside the block most are small: not tried.)
+    bool merging = d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0 && (growth > 0 || cut < 1024);
+    merge_tables mt[2];
+    if (merging) {
+        const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
+        std::exception_ptr failed;
+        std::thread back([&] {
+            try {
+                mt[1] = build_merged_levels(T_, true, L - c, L, d.b_levels, growth);
+            } catch (...) {
+                failed = std::current_exception();
+            }
+        });
+        try {
+            mt[0] = build_merged_levels(T_, false, 0, c, d.f_levels, growth);
+        } catch (...) {
+            back.join();
+            throw;
+        }
+        back.join();
+        if (failed) std::rethrow_exception(failed);
+        // Merged levels have no tail runs, which walk a small level in a quarter
+        // of a launch: a long chain of them outside the block (R-MAT scale 22:
+        // ~6,000 levels) is faster walked (fp64 solve 773 ms merged). By the
+        // factor alone, so that every schedule agrees on it.
+        double walked = 0;
+        for (int q = 0; q < c; ++q) walked += d.f_levels[q + 1] - d.f_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
+        for (int q = L - c; q < L; ++q) walked += d.b_levels[q + 1] - d.b_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
+        merging = growth > 0 || 4.5 * static_cast<double>(mt[0].steps.size() + mt[1].steps.size()) < walked;
+    }
     // Level tiles, the two directions side by side, where levels are not merged
     // (APXCHOL_AMD_TILE_LEVELS: levels a launch may join, 1: none). A solver for
     // one solve goes without: on a mixed 128^3 system they take 0.2 s and save
@@ -1264,24 +1300,6 @@ void gpu_solver::setup(const csc_view& L) {
     // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
     // may gain; 0: no merging).
     if (merging) {
-        const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
-        merge_tables mt[2];
-        std::exception_ptr failed;
-        std::thread back([&] {
-            try {
-                mt[1] = build_merged_levels(T_, true, L - c, L, d.b_levels, growth);
-            } catch (...) {
-                failed = std::current_exception();
-            }
-        });
-        try {
-            mt[0] = build_merged_levels(T_, false, 0, c, d.f_levels, growth);
-        } catch (...) {
-            back.join();
-            throw;
-        }
-        back.join();
-        if (failed) std::rethrow_exception(failed);
         for (int dir = 0; dir < 2; ++dir) {
             merge_tables& t = mt[dir];
             d.plan[dir] = t.steps;

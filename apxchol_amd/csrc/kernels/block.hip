@@ -609,9 +609,61 @@ __global__ __launch_bounds__(kBlock) void spmm_sell_staged_k(sell_desc a, int kp
     col_block_partials<1>(v, kp, part, sh);
 }
 
+// Long rows [first, a.nlong) of the SpMM for KP >= 4 columns, one wave per row:
+// thread (h, c) sums column c of the chains i * 64 / KP + h, i < KP, of
+// long_row_sum's 64 lanes, so an entry's KP gathers are contiguous (a wave per
+// column gathers a line per value); the chains are then added in wave_sum's
+// order, first in registers, then across lanes: the single SpMV's bits.
+template <class VT, int KP>
+__global__ __launch_bounds__(kBlock) void spmm_long_k(sell_desc a, int first, const double* __restrict__ x,
+                                                      double* __restrict__ y, const batch_state* bs) {
+    if (bs->active == 0) return;
+    constexpr int H = kWave / KP, U = KP < 8 ? KP : 8;
+    const int lane = threadIdx.x & (kWave - 1);
+    const int c = lane & (KP - 1), h = lane / KP;
+    const VT* __restrict__ cval = static_cast<const VT*>(a.cval);
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(blockIdx.x) * kWavesPerBlock +
+                                                    static_cast<int>(threadIdx.x) / kWave);
+    for (int li = first + wave; li < a.nlong; li += static_cast<int>(gridDim.x) * kWavesPerBlock) {
+        const int row = a.longrows[li];
+        const unsigned b = a.ptr[row], e = a.ptr[row + 1];
+        double s[KP];
+#pragma unroll
+        for (int i = 0; i < KP; ++i) s[i] = 0.0;
+        for (unsigned p = b; p < e; p += kWave) {
+#pragma unroll
+            for (int i0 = 0; i0 < KP; i0 += U) {
+                int j[U];
+                VT v[U];
+                double g[U];
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const unsigned q = p + static_cast<unsigned>((i0 + u) * H + h);
+                    j[u] = a.cidx[q < e ? q : b];
+                    v[u] = cval[q < e ? q : b];
+                }
+#pragma unroll
+                for (int u = 0; u < U; ++u) g[u] = x[static_cast<size_t>(j[u]) * KP + c];
+#pragma unroll
+                for (int u = 0; u < U; ++u)
+                    if (p + static_cast<unsigned>((i0 + u) * H + h) < e)
+                        s[i0 + u] = fma(static_cast<double>(v[u]), g[u], s[i0 + u]);
+            }
+        }
+#pragma unroll
+        for (int off = KP / 2; off >= 1; off >>= 1)
+#pragma unroll
+            for (int i = 0; i < off; ++i) s[i] += s[i + off];
+        double t = s[0];
+#pragma unroll
+        for (int off = H / 2; off >= 1; off >>= 1) t += __shfl_xor(t, off * KP, kWave);
+        if (h == 0) y[static_cast<size_t>(row) * KP + c] = t;
+    }
+}
+
 // p.Ap over the long rows of the sliced-ELL form, per column in long-row
-// order, stored as one more block of partials (block nb, after
-// spmm_sell_k's): a column's total does not depend on its slot.
+// order, stored as further blocks of partials (from nb on, after the SpMM's):
+// a column's total does not depend on its slot.
 __global__ __launch_bounds__(kBlock) void spmm_long_dot_k(sell_desc a, int kp, const double* __restrict__ x,
                                                           const double* __restrict__ y, const batch_state* bs,
                                                           double* part, int nb) {
@@ -620,7 +672,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_dot_k(sell_desc a, int kp, c
     const int c = threadIdx.x & (kp - 1);
     const int j = threadIdx.x / kp, rows = kBlock / kp;
     double s = 0.0;
-    for (int i = j; i < a.nlong; i += rows) {
+    for (int i = static_cast<int>(blockIdx.x) * rows + j; i < a.nlong; i += static_cast<int>(gridDim.x) * rows) {
         const size_t o = static_cast<size_t>(a.longrows[i]) * kp + c;
         s = fma(x[o], y[o], s);
     }
@@ -629,7 +681,7 @@ __global__ __launch_bounds__(kBlock) void spmm_long_dot_k(sell_desc a, int kp, c
     if (threadIdx.x < kp) {
         double t = sh[c];
         for (int r = 1; r < rows; ++r) t += sh[r * kp + c];
-        part[col_part(nb, 0, c, kp)] = t;
+        part[col_part(nb + static_cast<int>(blockIdx.x), 0, c, kp)] = t;
     }
 }
 

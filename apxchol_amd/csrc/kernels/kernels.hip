@@ -747,11 +747,27 @@ void launch_spmm_k(int n, int kp, int lanes, const unsigned* ptr, const int* idx
     if (want_dot) finish_k(kBFinPAp, n, kp, part, g, st, bs, s);
 }
 
-void launch_spmm_sell_k(const sell_desc& a, bool val32, int kp, const double* x, double* y, pcg_state* st,
+template <class VT>
+static void spmm_long(const sell_desc& a, int kp, const double* x, double* y, const batch_state* bs, hipStream_t s) {
+    const int waves = a.nlong - a.nhuge;
+    const int g = std::min((waves + kWavesPerBlock - 1) / kWavesPerBlock, 8192);
+    const auto f = kp == 4    ? spmm_long_k<VT, 4>
+                   : kp == 8  ? spmm_long_k<VT, 8>
+                   : kp == 16 ? spmm_long_k<VT, 16>
+                   : kp == 32 ? spmm_long_k<VT, 32>
+                              : spmm_long_k<VT, 64>;
+    f<<<g, kBlock, 0, s>>>(a, a.nhuge, x, y, bs);
+    check_launch("spmm_long_k");
+}
+
+void launch_spmm_sell_k(const sell_desc& op, bool val32, int kp, const double* x, double* y, pcg_state* st,
                         batch_state* bs, double* part, bool want_dot, hipStream_t s) {
     check_kp(kp);
-    const long long items = (static_cast<long long>(a.nslices) + a.nlong) * kp;
-    if (items <= 0) return;
+    if ((static_cast<long long>(op.nslices) + op.nlong) <= 0) return;
+    // From 4 columns on all but the huge long rows run in a launch of their own.
+    sell_desc a = op;
+    if (kp >= 4) a.nlong = op.nhuge;
+    const long long items = std::max(1ll, (static_cast<long long>(a.nslices) + a.nlong) * kp);
     long long g = (items + kWavesPerBlock - 1) / kWavesPerBlock;
     if (g > vec_block_cap()) g = vec_block_cap();
     g = std::max<long long>(kXcds, g / kXcds * kXcds);
@@ -773,14 +789,20 @@ void launch_spmm_sell_k(const sell_desc& a, bool val32, int kp, const double* x,
         else spmm_sell_k<double><<<grid, kBlock, 0, s>>>(a, kp, x, y, bs, part, w);
         check_launch("spmm_sell_k");
     }
+    if (op.nlong > a.nlong) {
+        if (val32) spmm_long<float>(op, kp, x, y, bs, s);
+        else spmm_long<double>(op, kp, x, y, bs, s);
+    }
     if (!want_dot) return;
     int nb = static_cast<int>(g);
-    if (a.nlong > 0) {
-        spmm_long_dot_k<<<1, kBlock, 0, s>>>(a, kp, x, y, bs, part, nb);
+    if (op.nlong > 0) {
+        const long long most = static_cast<long long>(op.nlong) * kp / (16 * kBlock);
+        const int blocks = static_cast<int>(std::clamp<long long>(most, 1, kLongDotBlocks));
+        spmm_long_dot_k<<<blocks, kBlock, 0, s>>>(op, kp, x, y, bs, part, nb);
         check_launch("spmm_long_dot_k");
-        ++nb;
+        nb += blocks;
     }
-    finish_k(kBFinPAp, a.n, kp, part, nb, st, bs, s);
+    finish_k(kBFinPAp, op.n, kp, part, nb, st, bs, s);
 }
 
 void launch_scatter_init_k(int n, int k, int kp, const unsigned* perm, const double* B, double* r, double* x,

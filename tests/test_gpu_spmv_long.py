@@ -47,3 +47,27 @@ def test_rows_at_round_edges(gpu, degree, monkeypatch):
         assert np.all(np.abs(y - A @ X[c]) <= 1e-13 * bound)
         assert np.array_equal(y.view(np.int64), Y[c].view(np.int64)), c
     s.close()
+
+
+@pytest.mark.parametrize("k", [1, 2, 4, 7, 16, 32, 33])
+@pytest.mark.parametrize("degree", [65, 1024, 1025, 1500])
+def test_block_widths_on_both_sides_of_the_huge_rows(gpu, degree, k, monkeypatch):
+    """A long row of up to 1024 entries (of these few) is summed by one wave for
+    all columns, a longer one by a wave per column: each column the single
+    product's bits at every block width, and a blocked solve converges."""
+    import torch
+    print(f"[case] huge rows degree={degree} k={k}", flush=True)
+    A = hub_graph(degree, max(600, degree + 40))
+    monkeypatch.setenv("APXCHOL_AMD_SPMV", "sell")
+    s = ax.Solver(A, seed=0, precision="fp64")
+    X = np.random.default_rng(2).standard_normal((k, A.shape[0]))
+    Xd = torch.tensor(X, device=gpu)
+    Y = s.spmv_batch(Xd).cpu().numpy()
+    for c in range(k):
+        y = s.spmv(Xd[c].clone()).cpu().numpy()
+        assert np.array_equal(y.view(np.int64), Y[c].view(np.int64)), c
+    Z, infos = s.solve_batch(Xd, tol=1e-8)
+    for c in range(k):
+        z = Z[c].cpu().numpy()
+        assert np.linalg.norm(X[c] - A @ z) <= 2e-8 * np.linalg.norm(X[c])
+    s.close()
