@@ -1400,7 +1400,11 @@ bool gpu_solver::build_trail(std::uint32_t first) {
                        a.as<double>(), x.as<double>(), d.tr_s.get(), values, np, bad.as<int>(), nullptr);
     int flag = 0;
     hip_check(hipMemcpy(&flag, bad.get(), sizeof flag, hipMemcpyDeviceToHost), "trailing block");
-    if (flag != 0) {   // an inverse outside the vectors' range: the levels are walked
+    std::vector<double> s_diag(static_cast<std::size_t>(n));
+    hip_check(hipMemcpy(s_diag.data(), a.get(), s_diag.size() * sizeof(double), hipMemcpyDeviceToHost), "trailing block");
+    // An inverse outside the vectors' range, or one that its rounding could
+    // spoil: the levels are walked.
+    if (flag != 0 || !trail_is_sound(T_, first, s_diag)) {
         d.tr_s.alloc(0);
         return false;
     }

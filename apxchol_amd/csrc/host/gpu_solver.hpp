@@ -270,7 +270,8 @@ private:
               int* defer = nullptr) const;
     void enqueue_precondition(bool first, int step, hipStream_t s) const;
     // Forms the trailing block of the rows from `first` on; false (and no
-    // block) when its inverse leaves the vectors' range.
+    // block) when its inverse leaves the vectors' range or its rounding could
+    // spoil it (trail_is_sound).
     bool build_trail(std::uint32_t first);
     // z = (L L^T)^-1 r in storage order: the forward levels, the trailing
     // block, the back levels; one vector, and kp columns of block `which`.

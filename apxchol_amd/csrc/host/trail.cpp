@@ -1,6 +1,7 @@
 #include "trail.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <stdexcept>
 
 namespace apxchol_amd {
@@ -44,6 +45,30 @@ constexpr std::uint32_t kMinFactorPerBlock = 6;
 // 18.2, against R-MAT s18 mixed 42.8 -> 9.8 and 89^3 fp64 18.6 -> 11.8.
 constexpr std::uint64_t kMinPerRow64 = 5, kMinPerRow32 = 10;
 
+// Largest sqrt(n) |D T|^2 of a block (trail_is_sound). A weak link between
+// clusters or a slight regularisation leaves S a large, nearly constant part,
+// whose rounding hides S's small eigenvalues; the walk, which rounds each row
+// once, is off by the square root of this only. The largest component of an
+// R-MAT graph of scale 11 (alone, with e on the diagonal, two of it joined by
+// an edge of weight w): sqrt(n) |D T|^2, the least eigenvalue of D^-1 S D^-1
+// exact and rounded to fp32, and iterations of mixed solves (N(0,1) projected,
+// 1e-8) walked and with S:
+//   alone            127     0.374    0.374
+//   e = 1e-2       9,800   5.1e-3   5.1e-3     11, 11, 11   11, 11, 11
+//   w = 1          2.4e5   2.7e-4   2.7e-4     13, 12, 11   12, 12, 11
+//   w = 1e-2       2.4e7  2.68e-6  2.67e-6     13, 12, 12   13, 12, 12
+//   e = 1e-6       1.0e8   4.4e-7  -8.2e-8     11, 10, 11   22, 22, 18
+//   w = 1e-3       2.4e8   2.7e-7  -2.5e-8     68, 13, 11   none converges
+//   e = 1e-8       1.0e10  4.4e-9  -2.9e-6     13, 13, 13   none converges
+// fp64 solves keep their iterations, but an application is further off: at the
+// limit S may be 7e-12 off (fp32: 0.4 %). Energy-norm errors of an application
+// to T times N(0,1), walked and with S: R-MAT s18 (13,000) 3e-15 / 3e-13,
+// w = 1 3e-15 / 3e-12, w = 1e-4 2e-13 / 2e-8. Blocks of grids (2-D up to
+// 1000, 3-D up to 112, anisotropic up to 80) have up to 3,300, of R-MAT graphs
+// of scale 11 to 22 up to 14,000.
+constexpr double kMaxSpread = 65536.0;
+constexpr int kSpreadSteps = 8;
+
 }  // namespace
 
 std::size_t choose_trail_level(const trsv_factor& T, int value_bytes, const std::vector<int>& fwd_first,
@@ -75,6 +100,55 @@ std::size_t choose_trail_level(const trsv_factor& T, int value_bytes, const std:
         }
     }
     return best;
+}
+
+// With D = sqrt(diag S) every |S_ij| is at most D_i D_j, so the rounding moves
+// x^T S x by at most u sqrt(n) |D x|^2 (its n^2 errors being independent), and
+// x^T S x is at least |D x|^2 / |D T|^2. The product of the two, u sqrt(n)
+// |D T|^2, bounds the relative change of the operator in its own norm. |D T|^2
+// is at most the largest eigenvalue of B B^T with B = |D T|, hence at most
+// max_i (B B^T v)_i / v_i for any v > 0: a few steps from v = 1 come within a
+// tenth of it.
+bool trail_is_sound(const trsv_factor& T, std::uint32_t first, const std::vector<double>& s_diag) {
+    const std::uint32_t n = T.m - first;
+    if (s_diag.size() < n) throw std::runtime_error("apxchol_amd: diagonal of the trailing block");
+    // B's rows: the block's entries, the diagonal last (columns of T over
+    // sqrt(W) where W is not 1).
+    std::vector<std::size_t> at(n + 1, 0);
+    std::vector<std::uint32_t> col;
+    std::vector<double> val;
+    for (std::uint32_t i = 0; i < n; ++i) {
+        if (!(s_diag[i] > 0.0) || !std::isfinite(s_diag[i])) return false;
+        const double d = std::sqrt(s_diag[i]);
+        const auto add = [&](std::uint32_t j, double v) {
+            col.push_back(j);
+            val.push_back(d * std::fabs(v) / (T.inv_scale.empty() ? 1.0 : static_cast<double>(T.inv_scale[first + j])));
+        };
+        for (std::uint32_t p = T.f_ptr[first + i]; p < T.f_ptr[first + i + 1]; ++p)
+            if (static_cast<std::uint32_t>(T.f_idx[p]) >= first)
+                add(static_cast<std::uint32_t>(T.f_idx[p]) - first, T.fp16 ? fp16_widen(T.f_h[p]) : T.f_val[p]);
+        add(i, T.diag[first + i]);
+        at[i + 1] = col.size();
+    }
+    std::vector<double> v(n, 1.0), w(n), t(n);
+    for (int step = 0; step < kSpreadSteps; ++step) {
+        std::fill(w.begin(), w.end(), 0.0);
+        for (std::uint32_t i = 0; i < n; ++i)
+            for (std::size_t k = at[i]; k < at[i + 1]; ++k) w[col[k]] += val[k] * v[i];
+        double most = 0.0, top = 0.0;
+        for (std::uint32_t i = 0; i < n; ++i) {
+            t[i] = 0.0;
+            for (std::size_t k = at[i]; k < at[i + 1]; ++k) t[i] += val[k] * w[col[k]];
+            const double q = t[i] / v[i];
+            if (!std::isfinite(q)) return false;
+            most = std::max(most, q);
+            top = std::max(top, t[i]);
+        }
+        if (std::sqrt(static_cast<double>(n)) * most <= kMaxSpread) return true;
+        // (Rows a step leaves far behind would divide by nothing.)
+        for (std::uint32_t i = 0; i < n; ++i) v[i] = std::max(t[i] / top, 1e-30);
+    }
+    return false;
 }
 
 trail_couple_tables build_trail_couple(const trsv_factor& T, std::uint32_t first) {

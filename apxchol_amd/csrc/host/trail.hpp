@@ -17,6 +17,11 @@ namespace apxchol_amd {
 std::size_t choose_trail_level(const trsv_factor& T, int value_bytes, const std::vector<int>& fwd_first,
                                const std::vector<int>& bck_first, int max_rows = -1);
 
+// Whether S = T^-T W T^-1 of the rows from `first` on, each entry rounded to
+// the sweeps' vector type, may stand for the walk of those rows. s_diag: S's
+// diagonal before the rounding.
+bool trail_is_sound(const trsv_factor& T, std::uint32_t first, const std::vector<double>& s_diag);
+
 // The entries of the rows [first, m) that lie before `first`, for
 // trail_couple: rows of at most 64 * kEpl of them in lane batches, the others
 // listed with their range in the forward lists.

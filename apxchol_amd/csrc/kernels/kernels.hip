@@ -557,8 +557,8 @@ void launch_trail_setup(const sweep_desc& fwd, const float* inv_scale, vec_prec 
     }
     const dim3 g(static_cast<unsigned>(np / kWave), static_cast<unsigned>(np / kWave));
     const float* w = inv_scale ? inv_scale + first : nullptr;
-    if (p == vec_prec::fp64) trail_form<double><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<double*>(s), ld, bad);
-    else trail_form<float><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<float*>(s), ld, bad);
+    if (p == vec_prec::fp64) trail_form<double><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<double*>(s), ld, a, bad);
+    else trail_form<float><<<g, kBlock, 0, st>>>(n, np, x, w, static_cast<float*>(s), ld, a, bad);
     check_launch("trail_setup");
 }
 

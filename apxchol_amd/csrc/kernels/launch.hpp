@@ -119,8 +119,9 @@ int trail_blocks(const trail_desc& t, vec_prec p);
 std::size_t trail_lds(const trail_desc& t, vec_prec p);
 int trail_couple_blocks(const trail_desc& t);
 // Forms S of the rows [first, first + n) of the factor: a, x are scratch of
-// np * np doubles (np: n rounded up to 64), s the zero-filled output; *bad
-// becomes non-zero when an entry is not finite.
+// np * np doubles (np: n rounded up to 64), s the output; a then starts with
+// S's diagonal before its rounding; *bad becomes non-zero when an entry is not
+// finite.
 void launch_trail_setup(const sweep_desc& fwd, const float* inv_scale, vec_prec p, bool fp16, int first, int n, int np,
                         double* a, double* x, void* s, std::size_t s_values, int ld, int* bad, hipStream_t st);
 

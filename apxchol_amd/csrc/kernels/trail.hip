@@ -15,8 +15,10 @@
 // block's levels in both directions is one coupling launch and one symmetric
 // matrix-vector product. S is computed once per factor, in fp64 on the matrix
 // cores, and kept in the sweeps' vector precision. Every entry of T_^-1 is a
-// sum of terms of one sign (the factor's off-diagonals are never positive),
-// so the inverse carries no cancellation. c and the product's sums are fp64
+// sum of terms of one sign (the factor's off-diagonals are never positive), so
+// forming S cancels nothing; rounding its entries does hide what a much softer
+// direction covers, and a factor where that could matter walks every level
+// (trail_is_sound, host/trail.cpp). c and the product's sums are fp64
 // for fp32 vectors too: fp32 sums of a few thousand terms of both signs lost
 // digits the walked levels keep (256^2 grid, projected N(0,1), error of an
 // application against fp64: walked 8.5e-7, fp32 sums 1.5e-6, fp64 sums 3.9e-7;
@@ -398,11 +400,13 @@ __global__ __launch_bounds__(kBlock) void trail_invert_step(int np, int s, int s
 }
 
 // S = X^T W X, the lower tiles and their mirror image, in the sweeps' vector
-// precision, with zeros in the padding (rows and columns past n); raises
-// bad on an entry that is not finite. Grid: (np / 64, np / 64).
+// precision, with zeros in the padding (rows and columns past n), and S's
+// diagonal as formed; raises bad on an entry that is not finite. Grid:
+// (np / 64, np / 64).
 template <class TO>
 __global__ __launch_bounds__(kBlock) void trail_form(int n, int np, const double* __restrict__ x,
-                                                     const float* __restrict__ w, TO* s, int ld, int* bad) {
+                                                     const float* __restrict__ w, TO* s, int ld, double* diag,
+                                                     int* bad) {
     __shared__ double la[16][kTrailPad], lb[16][kTrailPad];
     const int i0 = static_cast<int>(blockIdx.y) * kWave, j0 = static_cast<int>(blockIdx.x) * kWave;
     if (j0 > i0) return;
@@ -412,6 +416,7 @@ __global__ __launch_bounds__(kBlock) void trail_form(int n, int np, const double
     trail_tile_each(t, [&](int i, int j, double v) {
         const int r = i0 + i, c = j0 + j;
         if (c > r) return;   // the mirror of an element below the diagonal
+        if (c == r && r < n) diag[r] = v;
         const TO o = (r < n && c < n) ? static_cast<TO>(v) : static_cast<TO>(0);
         if (!(fabs(static_cast<double>(o)) <= 1.0e300) || (sizeof(TO) == 4 && !(fabsf(static_cast<float>(o)) <= 3.0e38f)))
             atomicOr(bad, 1);
