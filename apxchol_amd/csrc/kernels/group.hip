@@ -167,7 +167,7 @@ __global__ __launch_bounds__(kCoupleThreads) void group_trail_couple(const group
 }
 
 template <class TO>
-__global__ __launch_bounds__(kTrailThreads) void group_trail_apply(const group_trail* __restrict__ units,
+__global__ __launch_bounds__(kTrailThreads, 8) void group_trail_apply(const group_trail* __restrict__ units,
                                                                    const int* __restrict__ starts, int count) {
     extern __shared__ unsigned char group_trail_lds[];
     const int b = static_cast<int>(blockIdx.x);

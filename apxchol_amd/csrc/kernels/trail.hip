@@ -30,6 +30,8 @@
 // schedules keep agreeing bit for bit.
 #include "common.hpp"
 
+#include <type_traits>
+
 namespace apxchol_amd {
 
 // ---- application ---------------------------------------------------------------
@@ -121,6 +123,16 @@ __global__ __launch_bounds__(kCoupleThreads) void trail_couple(trail_desc t, swe
                                bs);
 }
 
+// One term of the product without the zeros of S, which join rows of different
+// components: a workgroup one of whose sums is not finite sums again with it
+// (the same chains, an entry at a time: few registers), so an infinity or NaN
+// stays in its component as in the walk of the levels.
+template <class TO>
+__device__ __forceinline__ double trail_skip(TO v, double c, double acc) {
+    return v == static_cast<TO>(0) ? acc : fma(static_cast<double>(v), c, acc);
+}
+__device__ __forceinline__ bool trail_finite(double v) { return fabs(v) <= 1.7976931348623157e308; }
+
 // z_T = S c. HBM-bound: S is read once, n^2 values (R-MAT s18, 6,006 fp32
 // rows, 144 MB: 28.7 us, 5.0 TB/s, the rate of a plain copy; 256^2 grid, 1,551
 // fp64 rows, 19 MB: 8 us). With the coupling launch (31.6 us there: hub rows)
@@ -138,45 +150,73 @@ __device__ __forceinline__ void trail_apply_body(int vb, unsigned char* lds, con
     constexpr int kChunks = kTrailThreads / R;
     constexpr int kPerWave = kChunks / kTrailWaves;
     double* cs = reinterpret_cast<double*>(lds);
-    const int tid = static_cast<int>(threadIdx.x);
     const int ch = t.chunk;
-    for (int q = tid; q < kChunks * ch; q += kTrailThreads) cs[q] = q < t.n ? c[q] : 0.0;
-    __syncthreads();
-    const int p = tid / R;
-    const TO* __restrict__ s = static_cast<const TO*>(t.s) + static_cast<size_t>(p) * ch * t.ld + vb * R + tid % R;
-    const double* cp = cs + p * ch;
-    double acc = 0.0;
-    int k = 0;
-    for (; k + 16 <= ch; k += 16) {
-        TO v[16];
+    const auto product = [&](auto skip_zeros, int tid) {
+        for (int q = tid; q < kChunks * ch; q += kTrailThreads) cs[q] = q < t.n ? c[q] : 0.0;
+        __syncthreads();
+        const int p = tid / R;
+        const TO* __restrict__ s = static_cast<const TO*>(t.s) + static_cast<size_t>(p) * ch * t.ld + vb * R + tid % R;
+        const double* cp = cs + p * ch;
+        double acc = 0.0;
+        if constexpr (decltype(skip_zeros)::value) {
+#pragma unroll 1
+            for (int k = 0; k < ch; ++k) acc = trail_skip(s[static_cast<size_t>(k) * t.ld], cp[k], acc);
+        } else {
+            int k = 0;
+            for (; k + 16 <= ch; k += 16) {
+                TO v[16];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) v[u] = s[static_cast<size_t>(k + u) * t.ld];
+                for (int u = 0; u < 16; ++u) v[u] = s[static_cast<size_t>(k + u) * t.ld];
 #pragma unroll
-        for (int u = 0; u < 16; ++u) acc = fma(static_cast<double>(v[u]), cp[k + u], acc);
+                for (int u = 0; u < 16; ++u) acc = fma(static_cast<double>(v[u]), cp[k + u], acc);
+            }
+            for (; k < ch; k += 4) {
+                TO v[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) v[u] = s[static_cast<size_t>(k + u) * t.ld];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) acc = fma(static_cast<double>(v[u]), cp[k + u], acc);
+            }
+        }
+        __syncthreads();
+        cs[tid] = acc;
+        __syncthreads();
+        // The rows' sums are wave 0's.
+        static_assert(R <= kWave, "rows of a workgroup");
+        bool finite = true;
+        if (tid < R && vb * R + tid < t.n) {
+            double sum = 0.0;
+#pragma unroll
+            for (int w = 0; w < kTrailWaves; ++w) {
+                double q = cs[w * kWave + tid];
+#pragma unroll
+                for (int j = 1; j < kPerWave; ++j) q += cs[w * kWave + j * R + tid];
+                sum = w == 0 ? q : sum + q;
+            }
+            z[t.first + vb * R + tid] = static_cast<TO>(sum);
+            finite = trail_finite(sum);
+        }
+        return finite;
+    };
+    int tid = static_cast<int>(threadIdx.x);
+    const bool finite = product(std::false_type{}, tid);
+    // In cs, whose last reads are wave 0's too. (A variable of its own would
+    // move cs off its alignment: 8 to 10 us a product.)
+    int* again = reinterpret_cast<int*>(lds);
+    if (tid < kWave) {
+        const int any = __any(!finite);
+        if (tid == 0) *again = any;
     }
-    for (; k < ch; k += 4) {
-        TO v[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) v[u] = s[static_cast<size_t>(k + u) * t.ld];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) acc = fma(static_cast<double>(v[u]), cp[k + u], acc);
-    }
     __syncthreads();
-    cs[tid] = acc;
-    __syncthreads();
-    if (tid >= R || vb * R + tid >= t.n) return;
-    double sum = 0.0;
-#pragma unroll
-    for (int w = 0; w < kTrailWaves; ++w) {
-        double q = cs[w * kWave + tid];
-#pragma unroll
-        for (int j = 1; j < kPerWave; ++j) q += cs[w * kWave + j * R + tid];
-        sum = w == 0 ? q : sum + q;
+    if (*again) {
+        __syncthreads();
+        asm volatile("" : "+v"(tid));   // nothing of the first pass is kept for this one
+        (void)product(std::true_type{}, tid);
     }
-    z[t.first + vb * R + tid] = static_cast<TO>(sum);
 }
+// (Eight waves a SIMD: two workgroups a compute unit, 64 registers.)
 template <class TO>
-__global__ __launch_bounds__(kTrailThreads) void trail_apply(trail_desc t, const double* __restrict__ c,
+__global__ __launch_bounds__(kTrailThreads, 8) void trail_apply(trail_desc t, const double* __restrict__ c,
                                                              TO* __restrict__ z, const pcg_state* st) {
     extern __shared__ unsigned char trail_smem[];
     trail_apply_body<TO>(static_cast<int>(blockIdx.x), trail_smem, t, c, z, st);
@@ -200,47 +240,82 @@ __global__ __launch_bounds__(kTrailThreads) void trail_apply_k(trail_desc t, con
     const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int i = static_cast<int>(blockIdx.x) * kWave + lane;   // < ld: rows past n are zero in S
     const int c0 = static_cast<int>(blockIdx.y) * CT;
-    double q[CT];
+    // Output o of this workgroup is row blockIdx.x * kWave + o % kWave of column
+    // c0 + o / kWave; this thread's are every kTrailThreads-th.
+    constexpr int kOut = (kWave * CT + kTrailThreads - 1) / kTrailThreads;
+    double sum[kOut];
+    const auto row_of = [&](int x) {
+        const int o = static_cast<int>(threadIdx.x) + x * kTrailThreads;
+        const int row = static_cast<int>(blockIdx.x) * kWave + (o & (kWave - 1));
+        return o < kWave * CT && row < t.n ? row : -1;
+    };
+    // Returns whether every sum of this thread is finite.
+    const auto product = [&](auto skip_zeros) {
+        double q[CT];
 #pragma unroll
-    for (int j = 0; j < kPerWave; ++j) {
-        const int k0 = (w * kPerWave + j) * t.chunk;
-        const int k1 = min(k0 + t.chunk, t.n);
-        double acc[CT];
+        for (int j = 0; j < kPerWave; ++j) {
+            const int k0 = (w * kPerWave + j) * t.chunk;
+            const int k1 = min(k0 + t.chunk, t.n);
+            double acc[CT];
 #pragma unroll
-        for (int u = 0; u < CT; ++u) acc[u] = 0.0;
-        const TO* __restrict__ s = static_cast<const TO*>(t.s) + i;
-        int k = k0;
-        for (; k + 4 <= k1; k += 4) {
-            TO v[4];
+            for (int u = 0; u < CT; ++u) acc[u] = 0.0;
+            const TO* __restrict__ s = static_cast<const TO*>(t.s) + i;
+            int k = k0;
+            if constexpr (decltype(skip_zeros)::value) {
+#pragma unroll 1
+                for (; k < k1; ++k) {
+                    const TO v = s[static_cast<size_t>(k) * t.ld];
+                    const double* __restrict__ cr = c + static_cast<size_t>(k) * kp + c0;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) v[b] = s[static_cast<size_t>(k + b) * t.ld];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                const double* __restrict__ cr = c + static_cast<size_t>(k + b) * kp + c0;
-#pragma unroll
-                for (int u = 0; u < CT; ++u) acc[u] = fma(static_cast<double>(v[b]), cr[u], acc[u]);
+                    for (int u = 0; u < CT; ++u) acc[u] = trail_skip(v, cr[u], acc[u]);
+                }
             }
+            for (; k + 4 <= k1; k += 4) {
+                TO v[4];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) v[b] = s[static_cast<size_t>(k + b) * t.ld];
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const double* __restrict__ cr = c + static_cast<size_t>(k + b) * kp + c0;
+#pragma unroll
+                    for (int u = 0; u < CT; ++u) acc[u] = fma(static_cast<double>(v[b]), cr[u], acc[u]);
+                }
+            }
+            for (; k < k1; ++k) {
+                const TO v = s[static_cast<size_t>(k) * t.ld];
+                const double* __restrict__ cr = c + static_cast<size_t>(k) * kp + c0;
+#pragma unroll
+                for (int u = 0; u < CT; ++u) acc[u] = fma(static_cast<double>(v), cr[u], acc[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < CT; ++u) q[u] = j == 0 ? acc[u] : q[u] + acc[u];
         }
-        for (; k < k1; ++k) {
-            const TO v = s[static_cast<size_t>(k) * t.ld];
-            const double* __restrict__ cr = c + static_cast<size_t>(k) * kp + c0;
 #pragma unroll
-            for (int u = 0; u < CT; ++u) acc[u] = fma(static_cast<double>(v), cr[u], acc[u]);
+        for (int u = 0; u < CT; ++u) red[w][u][lane] = q[u];
+        __syncthreads();
+        bool finite = true;
+#pragma unroll
+        for (int x = 0; x < kOut; ++x) {
+            sum[x] = 0.0;
+            if (row_of(x) < 0) continue;
+            const int o = static_cast<int>(threadIdx.x) + x * kTrailThreads, rl = o & (kWave - 1), u = o / kWave;
+            sum[x] = red[0][u][rl];
+#pragma unroll
+            for (int v = 1; v < kTrailWaves; ++v) sum[x] += red[v][u][rl];
+            finite = finite && trail_finite(sum[x]);
         }
-#pragma unroll
-        for (int u = 0; u < CT; ++u) q[u] = j == 0 ? acc[u] : q[u] + acc[u];
-    }
-#pragma unroll
-    for (int u = 0; u < CT; ++u) red[w][u][lane] = q[u];
+        return finite;
+    };
+    __shared__ int again;
+    if (threadIdx.x == 0) again = 0;   // (a barrier of the product follows)
+    if (!product(std::false_type{})) again = 1;
     __syncthreads();
-    for (int o = static_cast<int>(threadIdx.x); o < kWave * CT; o += kTrailThreads) {
-        const int rl = o & (kWave - 1), u = o / kWave;
-        const int row = static_cast<int>(blockIdx.x) * kWave + rl;
-        if (row >= t.n) continue;
-        double sum = red[0][u][rl];
+    if (again) (void)product(std::true_type{});
 #pragma unroll
-        for (int v = 1; v < kTrailWaves; ++v) sum += red[v][u][rl];
-        z[static_cast<size_t>(t.first + row) * kp + c0 + u] = static_cast<TO>(sum);
+    for (int x = 0; x < kOut; ++x) {
+        if (row_of(x) < 0) continue;
+        const int u = (static_cast<int>(threadIdx.x) + x * kTrailThreads) / kWave;
+        z[static_cast<size_t>(t.first + row_of(x)) * kp + c0 + u] = static_cast<TO>(sum[x]);
     }
 }
 
