@@ -1364,7 +1364,8 @@ void gpu_solver::setup(const csc_view& L) {
                           &d.b_tlane, &d.b_tent, &d.b_tovf, &d.b_tovf_ent, &d.b_twalk, &d.f_tlane_r, &d.b_tlane_r,
                           &d.tail_val, &d.relabel, &d.tr_s, &d.tr_c, &d.tr_rec, &d.tr_ent, &d.tr_long,
                           &d.mg_rec[0], &d.mg_batch[0], &d.mg_idx[0], &d.mg_val[0], &d.mg_rec[1], &d.mg_batch[1],
-                          &d.mg_idx[1], &d.mg_val[1], &d.sell_soff,
+                          &d.mg_idx[1], &d.mg_val[1], &d.tile_rec[0], &d.tile_ent[0], &d.tile_rec[1], &d.tile_ent[1],
+                          &d.sell_soff,
                           &d.sell_idx, &d.sell_val, &d.sell_map, &d.sell_long})
         bytes += b->bytes();
     stats_.device_bytes = bytes;
@@ -1654,6 +1655,12 @@ void gpu_solver::single_collect(double* d_x, solve_result& res, hipStream_t s) c
 }
 
 // ---- blocked solves -----------------------------------------------------
+
+std::uint64_t gpu_solver::block_bytes(int kp) const {
+    const std::uint64_t n = static_cast<std::uint64_t>(std::max<std::int64_t>(n_, 1));
+    return static_cast<std::uint64_t>(kp) * sizeof(double) *
+           (6 * n + static_cast<std::uint64_t>(dev_->trail.n) + 2 * static_cast<std::uint64_t>(kColPartials));
+}
 
 // Block width for k columns (a power of two <= 64), with the block buffers
 // grown to it.

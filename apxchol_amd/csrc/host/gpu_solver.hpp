@@ -253,6 +253,9 @@ public:
     group_member_view group_view() const;
     const factorization& factor() const { return F_; }
     const trsv_factor& trsv() const { return T_; }
+    // Device bytes of a block session of kp columns beside stats().device_bytes:
+    // its r, x, p, Ap, y, z, the trailing block's input and the partials.
+    std::uint64_t block_bytes(int kp) const;
     const solver_stats& stats() const { return stats_; }
     std::int64_t rows() const { return n_; }
 

@@ -101,11 +101,10 @@ int solve_server::add(std::shared_ptr<gpu_solver> solver) {
     const int kp_small = small_slots > 0 && pow2(small_slots) < kp ? pow2(small_slots) : 0;
     const std::int64_t n = solver->rows();
     const std::uint64_t nn = static_cast<std::uint64_t>(std::max<std::int64_t>(n, 1));
-    // Solver arrays + each block (r, x, p, Ap, y, z and its b / x staging) +
-    // the single lane's b / x.
-    const std::uint64_t need = solver->stats().device_bytes +
-                               static_cast<std::uint64_t>(8) * nn * static_cast<std::uint64_t>(kp + kp_small) * sizeof(double) +
-                               static_cast<std::uint64_t>(2) * nn * sizeof(double);
+    // Solver arrays + each block with its b / x staging + the single lane's b / x.
+    const std::uint64_t need = solver->stats().device_bytes + solver->block_bytes(kp) +
+                               (kp_small > 0 ? solver->block_bytes(kp_small) : 0) +
+                               static_cast<std::uint64_t>(2) * nn * static_cast<std::uint64_t>(kp + kp_small + 1) * sizeof(double);
     auto ln = std::make_unique<lane>();
     {
         std::lock_guard<std::mutex> lk(mu_);
