@@ -34,6 +34,11 @@ void hip_check(hipError_t e, const char* what) {
     if (e != hipSuccess) throw std::runtime_error(std::string("apxchol_amd: ") + what + ": " + hipGetErrorString(e));
 }
 
+// Device memory that does not suffice.
+struct device_memory_error : std::runtime_error {
+    using std::runtime_error::runtime_error;
+};
+
 class dbuf {
 public:
     dbuf() = default;
@@ -43,9 +48,16 @@ public:
     dbuf& operator=(const dbuf&) = delete;
     void alloc(std::size_t bytes) {
         if (p_) { (void)hipFree(p_); p_ = nullptr; }
-        bytes_ = bytes;
+        bytes_ = 0;
         if (bytes == 0) return;
-        hip_check(hipMalloc(&p_, bytes), "hipMalloc");
+        const hipError_t e = hipMalloc(&p_, bytes);
+        if (e != hipSuccess) p_ = nullptr;
+        if (e == hipErrorOutOfMemory) {
+            (void)hipGetLastError();   // not the next launch's error
+            throw device_memory_error(std::string("apxchol_amd: hipMalloc: ") + hipGetErrorString(e));
+        }
+        hip_check(e, "hipMalloc");
+        bytes_ = bytes;
     }
     template <class T>
     void upload(const std::vector<T>& v) {
@@ -88,6 +100,16 @@ int env_int(const char* name, int dflt) {
 int env_flag(const char* name, int dflt) {
     const char* e = std::getenv(name);
     return (e && *e) ? std::atoi(e) : dflt;
+}
+
+// Device memory that a form of the sweeps beside their levels (the trailing
+// block with its setup, the merged levels, the level tiles) may take;
+// APXCHOL_AMD_EXTRA_BYTES lowers it. Where it does not suffice the solver does
+// without the form.
+void take_extra(std::uint64_t bytes) {
+    const char* e = std::getenv("APXCHOL_AMD_EXTRA_BYTES");
+    if (e && *e && bytes > std::strtoull(e, nullptr, 10))
+        throw device_memory_error("apxchol_amd: " + std::to_string(bytes) + " bytes past APXCHOL_AMD_EXTRA_BYTES");
 }
 
 int center_k_from_env() {
@@ -961,7 +983,15 @@ void gpu_solver::setup(const csc_view& L) {
     int trail_max = -1;
     if (const char* e = std::getenv("APXCHOL_AMD_TRAIL_ROWS"); e && *e) trail_max = std::max(0, std::atoi(e));
     std::size_t cut = choose_trail_level(T_, d.prec == vec_prec::fp64 ? 8 : 4, d.f_levels, d.b_levels, trail_max);
-    if (cut < L_all && !build_trail(T_.level_ptr[cut])) cut = L_all;
+    if (cut < L_all) {
+        bool formed = false;
+        try {
+            formed = build_trail(T_.level_ptr[cut]);
+        } catch (const device_memory_error&) {
+            for (dbuf* b : {&d.tr_s, &d.tr_rec, &d.tr_ent, &d.tr_long, &d.tr_c}) b->alloc(0);
+        }
+        if (!formed) cut = L_all;
+    }
     // What the level tiles of a direction are built from.
     struct tile_input {
         lane_tables lt;
@@ -1217,6 +1247,9 @@ void gpu_solver::setup(const csc_view& L) {
                d.f_level_pos, d.f_level_diag);
     make_sched(d.b_sched, bb, true, d.b_levels, d.b_levels_dev, d.b_seg, b_tb, d.b_level_lb, d.b_lrec, d.b_lent,
                d.b_level_pos, d.b_level_diag);
+    // An application's steps outside the trailing block, the two directions side
+    // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
+    // may gain; 0: no merging).
     long long growth = opts_.merge_levels ? -1 : 0;
     if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
     // (Of 1024 levels and more outside the block most are small: not tried.)
@@ -1249,6 +1282,15 @@ void gpu_solver::setup(const csc_view& L) {
         for (int q = L - c; q < L; ++q) walked += d.b_levels[q + 1] - d.b_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
         merging = growth > 0 || 4.5 * static_cast<double>(mt[0].steps.size() + mt[1].steps.size()) < walked;
     }
+    if (merging) {
+        try {
+            upload_merged(mt[0], mt[1]);
+        } catch (const device_memory_error&) {
+            merging = false;
+            for (int dir = 0; dir < 2; ++dir)
+                for (dbuf* b : {&d.mg_rec[dir], &d.mg_batch[dir], &d.mg_idx[dir], &d.mg_val[dir]}) b->alloc(0);
+        }
+    }
     // Level tiles, the two directions side by side, where levels are not merged
     // (APXCHOL_AMD_TILE_LEVELS: levels a launch may join, 1: none). A solver for
     // one solve goes without: on a mixed 128^3 system they take 0.2 s and save
@@ -1277,13 +1319,27 @@ void gpu_solver::setup(const csc_view& L) {
         }
         back.join();
         if (failed) std::rethrow_exception(failed);
+        try {
+            std::uint64_t total = 0;
+            for (const tile_input& t : tile_in)
+                total += t.out.rec.size() * sizeof(lane_rec) + t.out.ent.size() * sizeof(entry32);
+            take_extra(total);
+            for (int dir = 0; dir < 2; ++dir) {
+                d.tile_rec[dir].upload(tile_in[dir].out.rec);
+                d.tile_ent[dir].upload(tile_in[dir].out.ent);
+            }
+        } catch (const device_memory_error&) {
+            for (int dir = 0; dir < 2; ++dir) {
+                d.tile_rec[dir].alloc(0);
+                d.tile_ent[dir].alloc(0);
+                tile_in[dir].out.steps.clear();
+            }
+        }
         for (int dir = 0; dir < 2; ++dir) {
             sweep_sched& sc = dir ? d.b_sched : d.f_sched;
             tile_tables& t = tile_in[dir].out;
             d.tiles[dir] = std::move(t.steps);
             if (d.tiles[dir].empty()) continue;
-            d.tile_rec[dir].upload(t.rec);
-            d.tile_ent[dir].upload(t.ent);
             sc.tiles = d.tiles[dir].data();
             sc.ntiles = static_cast<int>(d.tiles[dir].size());
             sc.tile_rec_dev = d.tile_rec[dir].as<lane_rec>();
@@ -1294,41 +1350,6 @@ void gpu_solver::setup(const csc_view& L) {
                 if (cut == L_all || (dir ? x.level >= sc.cut_level : x.level < sc.cut_level))
                     stats_.solve_level_launches[dir] -= x.levels - 1;
             }
-        }
-    }
-    // An application's steps outside the trailing block, the two directions side
-    // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
-    // may gain; 0: no merging).
-    if (merging) {
-        for (int dir = 0; dir < 2; ++dir) {
-            merge_tables& t = mt[dir];
-            d.plan[dir] = t.steps;
-            d.mg_rec[dir].upload(t.rec);
-            d.mg_batch[dir].upload(t.batch);
-            d.mg_idx[dir].alloc(t.slots * sizeof(std::int32_t));
-            d.mg_val[dir].alloc(t.slots * sizeof(double));
-            std::size_t at = 0;
-            for (const auto& q : t.pieces) {
-                hip_check(hipMemcpy(d.mg_idx[dir].as<std::int32_t>() + at, q.idx.data(),
-                                    q.idx.size() * sizeof(std::int32_t), hipMemcpyHostToDevice), "upload");
-                hip_check(hipMemcpy(d.mg_val[dir].as<double>() + at, q.val.data(), q.val.size() * sizeof(double),
-                                    hipMemcpyHostToDevice), "upload");
-                at += q.idx.size();
-            }
-            sweep_sched& sc = dir ? d.b_sched : d.f_sched;
-            sc.planned = true;
-            sc.plan = d.plan[dir].data();
-            sc.nplan = static_cast<int>(d.plan[dir].size());
-            sc.merged.rec = d.mg_rec[dir].as<lane_rec>();
-            sc.merged.batch = d.mg_batch[dir].as<merge_batch>();
-            sc.merged.idx = d.mg_idx[dir].as<std::int32_t>();
-            sc.merged.val = d.mg_val[dir].as<double>();
-            sc.merged.batches = static_cast<int>(t.batch.size());
-            // An application launches its steps, no tail runs.
-            stats_.solve_level_bytes[dir] += stats_.solve_tail_bytes[dir];
-            stats_.solve_tail_bytes[dir] = 0;
-            stats_.solve_tail_runs[dir] = 0;
-            stats_.solve_level_launches[dir] = sc.nplan;
         }
     }
     // Coupling output, shared by the two directions (their sweeps never overlap).
@@ -1383,6 +1404,48 @@ void gpu_solver::setup(const csc_view& L) {
     setup_times_.sptrsv_setup_ms = ms_since(t_setup) - setup_times_.pcg_setup_ms;
 }
 
+void gpu_solver::upload_merged(const merge_tables& fwd, const merge_tables& bck) {
+    auto& d = *dev_;
+    std::uint64_t total = 0;
+    for (const merge_tables* t : {&fwd, &bck})
+        total += t->slots * (sizeof(std::int32_t) + sizeof(double)) + t->rec.size() * sizeof(lane_rec) +
+                 t->batch.size() * sizeof(merge_batch);
+    take_extra(total);
+    for (int dir = 0; dir < 2; ++dir) {
+        const merge_tables& t = dir ? bck : fwd;
+        d.mg_rec[dir].upload(t.rec);
+        d.mg_batch[dir].upload(t.batch);
+        d.mg_idx[dir].alloc(t.slots * sizeof(std::int32_t));
+        d.mg_val[dir].alloc(t.slots * sizeof(double));
+        std::size_t at = 0;
+        for (const auto& q : t.pieces) {
+            hip_check(hipMemcpy(d.mg_idx[dir].as<std::int32_t>() + at, q.idx.data(), q.idx.size() * sizeof(std::int32_t),
+                                hipMemcpyHostToDevice), "upload");
+            hip_check(hipMemcpy(d.mg_val[dir].as<double>() + at, q.val.data(), q.val.size() * sizeof(double),
+                                hipMemcpyHostToDevice), "upload");
+            at += q.idx.size();
+        }
+    }
+    for (int dir = 0; dir < 2; ++dir) {
+        const merge_tables& t = dir ? bck : fwd;
+        d.plan[dir] = t.steps;
+        sweep_sched& sc = dir ? d.b_sched : d.f_sched;
+        sc.planned = true;
+        sc.plan = d.plan[dir].data();
+        sc.nplan = static_cast<int>(d.plan[dir].size());
+        sc.merged.rec = d.mg_rec[dir].as<lane_rec>();
+        sc.merged.batch = d.mg_batch[dir].as<merge_batch>();
+        sc.merged.idx = d.mg_idx[dir].as<std::int32_t>();
+        sc.merged.val = d.mg_val[dir].as<double>();
+        sc.merged.batches = static_cast<int>(t.batch.size());
+        // An application launches its steps, no tail runs.
+        stats_.solve_level_bytes[dir] += stats_.solve_tail_bytes[dir];
+        stats_.solve_tail_bytes[dir] = 0;
+        stats_.solve_tail_runs[dir] = 0;
+        stats_.solve_level_launches[dir] = sc.nplan;
+    }
+}
+
 bool gpu_solver::build_trail(std::uint32_t first) {
     auto& d = *dev_;
     const int n = static_cast<int>(T_.m - first);
@@ -1395,7 +1458,9 @@ bool gpu_solver::build_trail(std::uint32_t first) {
     t.ld = np;
     t.chunk = ((n + chunks - 1) / chunks + 3) / 4 * 4;
     const std::size_t values = static_cast<std::size_t>(chunks) * t.chunk * np;
-    dbuf a(static_cast<std::size_t>(np) * np * sizeof(double)), x(a.bytes()), bad(sizeof(double));
+    const std::size_t scratch = static_cast<std::size_t>(np) * np * sizeof(double);
+    take_extra(values * vsz + 2 * scratch);
+    dbuf a(scratch), x(scratch), bad(sizeof(double));
     d.tr_s.alloc(values * vsz);
     launch_trail_setup(d.fwd, T_.fp16 ? d.inv_scale.as<float>() : nullptr, d.prec, T_.fp16, t.first, n, np,
                        a.as<double>(), x.as<double>(), d.tr_s.get(), values, np, bad.as<int>(), nullptr);

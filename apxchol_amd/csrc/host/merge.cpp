@@ -140,8 +140,10 @@ merge_tables build_merged_levels(const trsv_factor& T, bool backward, int lo, in
         const double s = static_cast<double>(T.inv_scale[r]);
         return s * s;
     };
-    // Without merging no thread is needed.
-    const unsigned nthr = max_growth == 0 ? 1u : std::clamp(std::thread::hardware_concurrency(), 1u, 8u);
+    // Without merging no thread is needed. The threads' scratch (9 bytes a row
+    // each) stays under 256 MB.
+    const unsigned room = static_cast<unsigned>(std::min<std::uint64_t>(8, (256ull << 20) / (9ull * std::max(m, 1u))));
+    const unsigned nthr = max_growth == 0 ? 1u : std::max(1u, std::min(room, std::thread::hardware_concurrency()));
     team workers(nthr);
     std::vector<scratch> scr(nthr);
     open_step open;

@@ -52,3 +52,57 @@ def test_server_charges_every_block_buffer(gpu):
         small.close()
         o.close()
     s.close()
+
+
+def _bits(t):
+    import torch
+    return t.view(torch.int64)
+
+
+@pytest.mark.parametrize("graph", ["rmat", "grid3d", "grid2d"])
+@pytest.mark.parametrize("precision", ["fp64", "fp32"])
+def test_without_memory_for_the_extra_forms_levels_are_walked(gpu, graph, precision, monkeypatch):
+    """No room for the trailing block, the merged levels and the tiles (as a
+    full device would leave): the solver is made all the same and gives the bits
+    of one that is told to do without them."""
+    import torch
+    print(f"[case] no extra memory {graph} {precision}", flush=True)
+    A = {"rmat": lambda: mg.rmat_laplacian(12), "grid3d": lambda: mg.grid_laplacian((14, 13, 12)),
+         "grid2d": lambda: mg.grid_laplacian((70, 60))}[graph]()
+    F = ax.factorize(A, seed=0)
+    b = torch.tensor(mg.request_rhs(A, F.sddm, 1), device=gpu)
+    monkeypatch.setenv("APXCHOL_AMD_EXTRA_BYTES", "0")
+    s = ax.Solver(A, factor=F, precision=precision)
+    monkeypatch.delenv("APXCHOL_AMD_EXTRA_BYTES")
+    for name, value in (("TRAIL_ROWS", "0"), ("MERGE_GROWTH", "0"), ("TILE_LEVELS", "1")):
+        monkeypatch.setenv(f"APXCHOL_AMD_{name}", value)
+    plain = ax.Solver(A, factor=F, precision=precision)
+    z, zp = s.apply(b).clone(), plain.apply(b).clone()
+    r, rp = s.solve(b, tol=1e-8), plain.solve(b, tol=1e-8)
+    torch.cuda.synchronize()
+    assert s.info["block"] == plain.info["block"] and s.info["block"]["rows"] == 0
+    assert s.info["device_bytes"] == plain.info["device_bytes"]
+    assert r.iterations == rp.iterations and r.status == 1
+    assert torch.equal(_bits(z), _bits(zp)) and torch.equal(_bits(r.x), _bits(rp.x))
+
+
+def test_without_memory_for_merged_levels_the_block_stays(gpu, monkeypatch):
+    """Room for a block of up to 64 rows (100 KB with its setup), not for the
+    merged levels (more than 1 MB)."""
+    import torch
+    print("[case] no memory for merged levels", flush=True)
+    A = mg.add_excess(mg.grid_laplacian((16, 16, 16), "lognormal"))
+    F = ax.factorize(A, seed=0)
+    b = torch.tensor(mg.rhs(A.shape[0], 2), device=gpu)
+    monkeypatch.setenv("APXCHOL_AMD_TRAIL_ROWS", "64")
+    monkeypatch.setenv("APXCHOL_AMD_MERGE_GROWTH", "4000")
+    monkeypatch.setenv("APXCHOL_AMD_TILE_LEVELS", "1")
+    full = ax.Solver(A, factor=F)
+    monkeypatch.setenv("APXCHOL_AMD_EXTRA_BYTES", "1000000")
+    s = ax.Solver(A, factor=F)
+    monkeypatch.delenv("APXCHOL_AMD_EXTRA_BYTES")
+    monkeypatch.setenv("APXCHOL_AMD_MERGE_GROWTH", "0")
+    plain = ax.Solver(A, factor=F)
+    assert full.info["block"]["rows"] == s.info["block"]["rows"] > 0
+    assert s.info["block"] == plain.info["block"] != full.info["block"]
+    assert torch.equal(_bits(s.apply(b).clone()), _bits(plain.apply(b).clone()))
