@@ -18,11 +18,11 @@
 #include <cstring>
 #include <stdexcept>
 #include <string>
-#include <thread>
 
 #include "../device.hpp"
 #include "../kernels/launch.hpp"
 #include "merge.hpp"
+#include "threads.hpp"
 #include "tile.hpp"
 #include "trail.hpp"
 
@@ -1257,22 +1257,10 @@ void gpu_solver::setup(const csc_view& L) {
     merge_tables mt[2];
     if (merging) {
         const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
-        std::exception_ptr failed;
-        std::thread back([&] {
-            try {
-                mt[1] = build_merged_levels(T_, true, L - c, L, d.b_levels, growth);
-            } catch (...) {
-                failed = std::current_exception();
-            }
+        side_by_side(2, [&](int dir) {
+            mt[dir] = dir ? build_merged_levels(T_, true, L - c, L, d.b_levels, growth)
+                          : build_merged_levels(T_, false, 0, c, d.f_levels, growth);
         });
-        try {
-            mt[0] = build_merged_levels(T_, false, 0, c, d.f_levels, growth);
-        } catch (...) {
-            back.join();
-            throw;
-        }
-        back.join();
-        if (failed) std::rethrow_exception(failed);
         // Merged levels have no tail runs, which walk a small level in a quarter
         // of a launch: a long chain of them outside the block (R-MAT scale 22:
         // ~6,000 levels) is faster walked (fp64 solve 773 ms merged). By the
@@ -1297,28 +1285,12 @@ void gpu_solver::setup(const csc_view& L) {
     // 2.3 ms a solve.
     const int tile_levels = env_int("APXCHOL_AMD_TILE_LEVELS", opts_.merge_levels ? kTileMaxLevels : 1);
     if (tile_levels > 1 && !merging) {
-        const auto build = [&](int dir) {
+        side_by_side(2, [&](int dir) {
             tile_input& t = tile_in[dir];
             for (const auto& run : t.runs)
                 append_tiles(t.lt, dir != 0, static_cast<std::uint32_t>(m), dir ? d.b_levels : d.f_levels,
                              dir ? d.b_level_lb : d.f_level_lb, t.level_pos, run.first, run.second, tile_levels, t.out);
-        };
-        std::exception_ptr failed;
-        std::thread back([&] {
-            try {
-                build(1);
-            } catch (...) {
-                failed = std::current_exception();
-            }
         });
-        try {
-            build(0);
-        } catch (...) {
-            back.join();
-            throw;
-        }
-        back.join();
-        if (failed) std::rethrow_exception(failed);
         try {
             std::uint64_t total = 0;
             for (const tile_input& t : tile_in)

@@ -5,6 +5,8 @@
 #include <barrier>
 #include <exception>
 #include <functional>
+#include <mutex>
+#include <optional>
 #include <stdexcept>
 #include <thread>
 
@@ -63,25 +65,36 @@ struct scratch {
     std::vector<std::uint32_t> touched;
 };
 
-// A few threads that run one job after another.
+// A few threads that run one job after another: at most n with the calling
+// one, fewer where the process may not start that many.
 class team {
 public:
-    explicit team(unsigned n) : n_(n), gate_(static_cast<std::ptrdiff_t>(n)) {
-        for (unsigned w = 1; w < n; ++w) threads_.emplace_back([this, w] { loop(w); });
+    explicit team(unsigned n) {
+        const std::lock_guard<std::mutex> hold(counting_);   // the threads wait for their number
+        threads_.reserve(n);
+        try {
+            for (unsigned w = 1; w < n; ++w)
+                threads_.emplace_back([this, w] {
+                    { const std::lock_guard<std::mutex> wait(counting_); }
+                    loop(w);
+                });
+        } catch (...) {   // no thread, or no memory for one
+        }
+        gate_.emplace(static_cast<std::ptrdiff_t>(size()));
     }
     ~team() {
         job_ = nullptr;
-        gate_.arrive_and_wait();
+        gate_->arrive_and_wait();
         for (auto& t : threads_) t.join();
     }
-    unsigned size() const { return n_; }
+    unsigned size() const { return static_cast<unsigned>(threads_.size()) + 1; }
     // job(w) on every thread; rethrows the first exception.
     void run(const std::function<void(unsigned)>& job) {
         job_ = &job;
         failed_ = nullptr;
-        gate_.arrive_and_wait();
+        gate_->arrive_and_wait();
         call(0);
-        gate_.arrive_and_wait();
+        gate_->arrive_and_wait();
         if (failed_) std::rethrow_exception(failed_);
     }
 
@@ -95,14 +108,14 @@ private:
     }
     void loop(unsigned w) {
         for (;;) {
-            gate_.arrive_and_wait();
+            gate_->arrive_and_wait();
             if (!job_) return;
             call(w);
-            gate_.arrive_and_wait();
+            gate_->arrive_and_wait();
         }
     }
-    unsigned n_;
-    std::barrier<> gate_;
+    std::mutex counting_;
+    std::optional<std::barrier<>> gate_;
     const std::function<void(unsigned)>* job_ = nullptr;
     std::atomic<bool> taken_{false};
     std::exception_ptr failed_;
@@ -143,8 +156,8 @@ merge_tables build_merged_levels(const trsv_factor& T, bool backward, int lo, in
     // Without merging no thread is needed. The threads' scratch (9 bytes a row
     // each) stays under 256 MB.
     const unsigned room = static_cast<unsigned>(std::min<std::uint64_t>(8, (256ull << 20) / (9ull * std::max(m, 1u))));
-    const unsigned nthr = max_growth == 0 ? 1u : std::max(1u, std::min(room, std::thread::hardware_concurrency()));
-    team workers(nthr);
+    team workers(max_growth == 0 ? 1u : std::max(1u, std::min(room, std::thread::hardware_concurrency())));
+    const unsigned nthr = workers.size();
     std::vector<scratch> scr(nthr);
     open_step open;
     std::uint32_t p0 = 0;        // first position of the open step

@@ -7,10 +7,10 @@
 #include "tile.hpp"
 
 #include <algorithm>
-#include <exception>
 #include <numeric>
 #include <stdexcept>
-#include <thread>
+
+#include "threads.hpp"
 
 namespace apxchol_amd {
 namespace {
@@ -219,20 +219,10 @@ public:
         if (t.pos.size() < 4096) {
             write(0, s.tiles, slots[0]);
         } else {
-            std::exception_ptr failed[kThreads];
-            std::vector<std::thread> th;
-            for (int q = 0; q < kThreads; ++q)
-                th.emplace_back([&, q] {
-                    try {
-                        write(static_cast<int>(static_cast<long long>(s.tiles) * q / kThreads),
-                              static_cast<int>(static_cast<long long>(s.tiles) * (q + 1) / kThreads), slots[q]);
-                    } catch (...) {
-                        failed[q] = std::current_exception();
-                    }
-                });
-            for (auto& x : th) x.join();
-            for (const auto& x : failed)
-                if (x) std::rethrow_exception(x);
+            side_by_side(kThreads, [&](int q) {
+                write(static_cast<int>(static_cast<long long>(s.tiles) * q / kThreads),
+                      static_cast<int>(static_cast<long long>(s.tiles) * (q + 1) / kThreads), slots[q]);
+            });
         }
         s.slots = *std::max_element(slots, slots + kThreads);
         tt.steps.push_back(s);
