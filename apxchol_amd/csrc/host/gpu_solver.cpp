@@ -1281,8 +1281,9 @@ void gpu_solver::setup(const csc_view& L) {
     }
     // Level tiles, the two directions side by side, where levels are not merged
     // (APXCHOL_AMD_TILE_LEVELS: levels a launch may join, 1: none). A solver for
-    // one solve goes without: on a mixed 128^3 system they take 0.2 s and save
-    // 2.3 ms a solve.
+    // one solve goes without: on a mixed 128^3 system they take 80 ms and save
+    // 3 ms a solve. (Built at the first call that runs them they would cost a
+    // solver of blocked or grouped solves nothing, but a first solve 80 ms more.)
     const int tile_levels = env_int("APXCHOL_AMD_TILE_LEVELS", opts_.merge_levels ? kTileMaxLevels : 1);
     if (tile_levels > 1 && !merging) {
         side_by_side(2, [&](int dir) {
@@ -1293,12 +1294,21 @@ void gpu_solver::setup(const csc_view& L) {
         });
         try {
             std::uint64_t total = 0;
-            for (const tile_input& t : tile_in)
-                total += t.out.rec.size() * sizeof(lane_rec) + t.out.ent.size() * sizeof(entry32);
+            constexpr std::size_t rec_b = kWave * sizeof(lane_rec), ent_b = kWave * kEpl * sizeof(entry32);
+            for (const tile_input& t : tile_in) total += static_cast<std::uint64_t>(t.out.batches) * (rec_b + ent_b);
             take_extra(total);
             for (int dir = 0; dir < 2; ++dir) {
-                d.tile_rec[dir].upload(tile_in[dir].out.rec);
-                d.tile_ent[dir].upload(tile_in[dir].out.ent);
+                const tile_tables& t = tile_in[dir].out;
+                d.tile_rec[dir].alloc(static_cast<std::size_t>(t.batches) * rec_b);
+                d.tile_ent[dir].alloc(static_cast<std::size_t>(t.batches) * ent_b);
+                std::size_t at = 0;
+                for (const auto& q : t.pieces) {
+                    hip_check(hipMemcpy(d.tile_rec[dir].as<lane_rec>() + at * kWave, q.rec.get(), q.batches * rec_b,
+                                        hipMemcpyHostToDevice), "upload");
+                    hip_check(hipMemcpy(d.tile_ent[dir].as<entry32>() + at * kWave * kEpl, q.ent.get(), q.batches * ent_b,
+                                        hipMemcpyHostToDevice), "upload");
+                    at += q.batches;
+                }
             }
         } catch (const device_memory_error&) {
             for (int dir = 0; dir < 2; ++dir) {

@@ -7,6 +7,7 @@
 #include "tile.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <numeric>
 #include <stdexcept>
 
@@ -23,8 +24,8 @@ namespace {
 // lose 4 %, at four times it as well.
 constexpr double kLaunchUs = 3.6, kLevelUs = 0.8, kTileBatchUs = 0.11, kBatchUs = 0.001;
 constexpr int kUnits = 256;   // compute units
-// Tiles a trial looks at (all: 128^3 25.2 ms a solve and 0.17 s of host time;
-// 4: 26.0 ms, 0.13 s).
+// Tiles a trial looks at (128^3: a solve 25.4 ms; with all 25.2 and 40 ms more
+// of host time, with 4 26.0 and as much time).
 constexpr int kSampleTiles = 32;
 
 double launch_us(int levels, double batches, double tile_batches) {
@@ -47,7 +48,7 @@ public:
         const std::size_t n = static_cast<std::size_t>(lp[l1]) - p0_;
         head_.assign(n, -1);
         level_.assign(n, -1);
-        mark_.assign(n, 0);
+        for (scratch& x : scratch_) x.mark.assign(n, 0);
         owner_.assign(n, 0);
         lanes_.assign(n, 0);
         for (int q = l0; q < l1; ++q)
@@ -81,14 +82,20 @@ public:
 
     // Tiles of the levels [a, a + J) with at most `waves` batches a level; false
     // when a row's tile would have more. limit > 0: an estimate of t.us from the
-    // first tiles of the last level.
-    bool build(int a, int J, int waves, tiling& t, int limit = 0) {
+    // first tiles of the last level. Calls with another `place` (below kPlaces)
+    // may run beside each other.
+    static constexpr int kPlaces = 3;
+    static_assert(4 << (kPlaces - 1) == kTileWaves, "a place for each number of waves");
+    bool build(int a, int J, int waves, tiling& t, int limit = 0, int place = 0) {
         t = {};
+        std::vector<int>& mark = scratch_[place].mark;
+        std::vector<int>& undo = scratch_[place].undo;
+        int& stamp = scratch_[place].stamp;
         std::vector<std::uint32_t> cur[kTileMaxLevels], add, stack;
         long long cnt[kTileMaxLevels] = {}, more[kTileMaxLevels];
         const std::uint32_t from = static_cast<std::uint32_t>(lp_[a]) - p0_;
-        const int base = stamp_;
-        ++stamp_;
+        const int base = stamp;
+        ++stamp;
         bool open = false;
         const auto close = [&] {
             for (int p = 0; p < J; ++p) {
@@ -98,42 +105,42 @@ public:
                 cur[p].clear();
                 cnt[p] = 0;
             }
-            ++stamp_;
+            ++stamp;
             open = false;
         };
         // Rows of the last level first; then those of the levels before it
         // that no tile has reached.
         for (int q = a + J - 1; q >= a; --q)
             for (std::uint32_t i = static_cast<std::uint32_t>(lp_[q]) - p0_; i < static_cast<std::uint32_t>(lp_[q + 1]) - p0_; ++i) {
-                if (mark_[i] > base) continue;
+                if (mark[i] > base) continue;
                 for (;;) {
                     add.clear();
                     std::fill(more, more + J, 0);
                     const auto reach = [&](std::uint32_t j) {
-                        mark_[j] = stamp_;
+                        mark[j] = stamp;
                         add.push_back(j);
                         stack.push_back(j);
                         more[level_[j] - a] += lanes_[j];
                     };
                     // Marks of the tiles before this one are kept for undoing.
-                    undo_.clear();
-                    undo_.push_back(mark_[i]);
+                    undo.clear();
+                    undo.push_back(mark[i]);
                     reach(i);
                     while (!stack.empty()) {
                         const std::uint32_t x = stack.back();
                         stack.pop_back();
                         for (std::size_t k = dep_at_[x]; k < dep_at_[x + 1]; ++k) {
                             const std::uint32_t j = dep_[k];
-                            if (j < from || mark_[j] == stamp_) continue;
-                            undo_.push_back(mark_[j]);
+                            if (j < from || mark[j] == stamp) continue;
+                            undo.push_back(mark[j]);
                             reach(j);
                         }
                     }
                     bool fits = true;
                     for (int p = 0; p < J; ++p) fits = fits && cnt[p] + more[p] <= waves * kWave;
                     if (fits) break;
-                    for (std::size_t k = 0; k < add.size(); ++k) mark_[add[k]] = undo_[k];
-                    if (!open) { stamp_ += 1; return false; }
+                    for (std::size_t k = 0; k < add.size(); ++k) mark[add[k]] = undo[k];
+                    if (!open) { stamp += 1; return false; }
                     close();
                     if (limit > 0 && q == a + J - 1 && static_cast<int>(t.lanes.size()) >= limit * J) {
                         const std::uint32_t q0 = static_cast<std::uint32_t>(lp_[q]) - p0_;
@@ -165,19 +172,25 @@ public:
             s.base[p] = static_cast<int>(tt.batches);
             tt.batches += static_cast<long long>(s.tiles) * s.width[p];
         }
-        tt.rec.resize(static_cast<std::size_t>(tt.batches) * kWave, {-1, 0});
-        tt.ent.resize(static_cast<std::size_t>(tt.batches) * kWave * kEpl, {0, 0.0f});
+        // Written by the slices below, padding included: memory that one thread
+        // has touched first, or that grows with every step, takes most of the
+        // build (64^3: 97 of 128 ms).
+        tile_tables::piece out;
+        const long long first_batch = s.base[0];
+        out.batches = static_cast<std::size_t>(tt.batches - first_batch);
+        out.rec = std::make_unique_for_overwrite<lane_rec[]>(out.batches * kWave);
+        out.ent = std::make_unique_for_overwrite<entry32[]>(out.batches * kWave * kEpl);
         // The first tile that computes a row writes it.
-        const int done = ++stamp_;
+        ++step_;
         std::vector<char> own(t.pos.size());
         for (std::size_t k = 0; k < t.pos.size(); ++k) {
-            own[k] = owner_[t.pos[k]] < done;
-            owner_[t.pos[k]] = done;
+            own[k] = owner_[t.pos[k]] < step_;
+            owner_[t.pos[k]] = step_;
         }
         const std::uint32_t p0 = static_cast<std::uint32_t>(lp_[a]), np = static_cast<std::uint32_t>(lp_[a + J]) - p0;
         // Tiles [k0, k1): their own slots in the records and entries.
         const auto write = [&](int k0, int k1, int& slots) {
-            std::vector<std::int32_t> slot_of(np);
+            const auto slot_of = std::make_unique_for_overwrite<std::int32_t[]>(np);
             std::vector<std::size_t> rows;
             for (int k = k0; k < k1; ++k) {
                 int slot = 0;
@@ -190,14 +203,19 @@ public:
                         const int gx = lanes_[t.pos[x]], gy = lanes_[t.pos[y]];
                         return gx != gy ? gx > gy : x < y;
                     });
-                    long long at = (static_cast<long long>(s.base[p]) + static_cast<long long>(k) * s.width[p]) * kWave;
+                    const std::size_t b0 = static_cast<std::size_t>(s.base[p] - first_batch) +
+                                           static_cast<std::size_t>(k) * static_cast<std::size_t>(s.width[p]);
+                    const std::size_t b1 = b0 + static_cast<std::size_t>(s.width[p]);
+                    std::fill(out.rec.get() + b0 * kWave, out.rec.get() + b1 * kWave, lane_rec{-1, 0});
+                    std::fill(out.ent.get() + b0 * kWave * kEpl, out.ent.get() + b1 * kWave * kEpl, entry32{0, 0.0f});
+                    long long at = static_cast<long long>(b0) * kWave;
                     for (const std::size_t x : rows) {
                         const std::uint32_t i = t.pos[x];
                         slot_of[i + p0_ - p0] = slot;
                         for (int g = 0; g < lanes_[i]; ++g, ++at) {
                             const long long from = head_[i] + g;
                             const lane_rec& r = lt_.rec[static_cast<std::size_t>(from)];
-                            lane_rec& o = tt.rec[static_cast<std::size_t>(at)];
+                            lane_rec& o = out.rec[static_cast<std::size_t>(at)];
                             o.row = r.row;
                             o.info = r.info | static_cast<std::uint32_t>(slot) << kTileSlotShift | (own[x] ? kTileOwn : 0u);
                             const int nv = static_cast<int>((r.info >> 9) & 7u);
@@ -205,7 +223,7 @@ public:
                                 entry32 v = lt_.ent[entry_at(from, e)];
                                 const std::uint32_t pj = position(v.idx);
                                 if (pj >= p0) v.idx = ~slot_of[pj - p0];
-                                tt.ent[entry_at(at, e)] = v;
+                                out.ent[entry_at(at, e)] = v;
                             }
                         }
                         ++slot;
@@ -226,6 +244,7 @@ public:
         }
         s.slots = *std::max_element(slots, slots + kThreads);
         tt.steps.push_back(s);
+        tt.pieces.push_back(std::move(out));
     }
 
 private:
@@ -265,8 +284,13 @@ private:
     std::vector<unsigned char> lanes_;   // lanes of the row
     std::vector<std::size_t> dep_at_;
     std::vector<std::uint32_t> dep_;
-    std::vector<int> level_, mark_, owner_, undo_;
-    int stamp_ = 1;
+    std::vector<int> level_, owner_;
+    int step_ = 0;
+    struct alignas(64) scratch {
+        std::vector<int> mark, undo;
+        int stamp = 1;
+    };
+    scratch scratch_[kPlaces];
 };
 
 }  // namespace
@@ -282,18 +306,24 @@ void append_tiles(const lane_tables& lt, bool backward, std::uint32_t m, const s
     // have become a third smaller or larger.
     int J = 0, waves = 0, at = 0;
     for (int l = l0; l + 1 < l1;) {
-        tiling keep, t;
+        tiling keep;
         if (at == 0 || 3 * std::abs(batches(l) - at) > at || l + J > l1 || (J > 1 && !T.build(l, J, waves, keep))) {
             at = std::max(1, batches(l));
             J = 1;
             double least = launch_us(1, batches(l), 0);
-            for (int j = 2; j <= std::min(max_levels, l1 - l) && j <= J + 1; ++j)
-                for (int w = 4; w <= kTileWaves; w *= 2)
-                    if (T.build(l, j, w, t, kSampleTiles) && t.us / j < least) {
-                        least = t.us / j;
+            for (int j = 2; j <= std::min(max_levels, l1 - l) && j <= J + 1; ++j) {
+                double us[tiler::kPlaces];
+                side_by_side(tiler::kPlaces, [&](int k) {
+                    tiling t;
+                    us[k] = T.build(l, j, 4 << k, t, kSampleTiles, k) ? t.us : HUGE_VAL;
+                });
+                for (int k = 0; k < tiler::kPlaces; ++k)
+                    if (us[k] / j < least) {
+                        least = us[k] / j;
                         J = j;
-                        waves = w;
+                        waves = 4 << k;
                     }
+            }
             if (J > 1 && !T.build(l, J, waves, keep)) J = 1;
         }
         if (J > 1) T.emit(l, J, keep, tt);

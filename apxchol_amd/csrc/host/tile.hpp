@@ -1,13 +1,21 @@
 // Level tiles of the launched levels (kernels/tile.hip): the host side.
 #pragma once
 
+#include <memory>
+
 #include "gpu_solver.hpp"
 
 namespace apxchol_amd {
 
 struct tile_tables {
-    std::vector<lane_rec> rec;     // batches of 64 lanes, step by step and level by level
-    std::vector<entry32> ent;      // kEpl planes of 64 per batch
+    // One piece a step, level by level in it: 64 lanes and kEpl planes of 64
+    // entries a batch.
+    struct piece {
+        std::size_t batches = 0;
+        std::unique_ptr<lane_rec[]> rec;
+        std::unique_ptr<entry32[]> ent;
+    };
+    std::vector<piece> pieces;
     long long batches = 0;
     std::vector<tile_step> steps;  // ascending levels, disjoint
 };
