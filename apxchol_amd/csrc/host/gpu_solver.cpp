@@ -1558,10 +1558,11 @@ void gpu_solver::enqueue_iteration(int it, hipStream_t s) const {
     enqueue_precondition(false, it, s);
 }
 
-int iterations_ahead(int least, double residual, std::int64_t iterations, double tol) {
-    if (!(residual > tol) || !(residual < 1.0) || !(tol > 0.0) || iterations < 1) return least;
+int iterations_ahead(int every, double residual, std::int64_t iterations, double tol) {
+    if (every != kItersPerCheck) return every;
+    if (!(residual > tol) || !(residual < 1.0) || !(tol > 0.0) || iterations < 1) return every;
     const double left = std::log(tol / residual) / std::log(residual) * static_cast<double>(iterations);
-    return std::max(least, static_cast<int>(std::min(0.5 * left, 32.0)));
+    return std::max(every, static_cast<int>(std::min(0.5 * left, 32.0)));
 }
 
 solve_result gpu_solver::solve_device(const double* d_b, double* d_x, double tol, int max_iter, const double* d_x0,

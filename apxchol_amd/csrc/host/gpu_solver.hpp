@@ -20,6 +20,9 @@ enum class sweep_precision { fp64 = 0, fp32 = 1 };   // vector / accumulation wi
 enum class sweep_schedule { dataflow = 0, levels = 1, hybrid = 2 };
 
 // solve.h:13-25 plus the device knobs.
+// Default of iters_per_check.
+inline constexpr int kItersPerCheck = 2;
+
 struct solve_options {
     double tol = 1e-8;
     int max_iter = 200;
@@ -34,7 +37,7 @@ struct solve_options {
     int tail_cut = 0;             // hybrid: a run ends before a level needing this many overflow groups per lane
                                   // (0: APXCHOL_AMD_TAIL_CUT or 1; < 0: never)
     double drop_rel = -1.0;       // < 0: APXCHOL_FACTOR_DROP / the 1e-4 default
-    int iters_per_check = 2;      // iterations enqueued between completion tests
+    int iters_per_check = kItersPerCheck;   // iterations enqueued between completion tests (iterations_ahead)
     int sweep_chunk = 0;          // batches per dataflow ticket (0: APXCHOL_AMD_SWEEP_CHUNK or 8)
     int sweep_blocks = 0;         // dataflow grid (0: APXCHOL_AMD_SWEEP_BLOCKS or the resident grid)
     bool graph = true;            // replay each PCG iteration as one captured HIP graph
@@ -101,11 +104,12 @@ struct solver_stats {
 struct block_sched;
 struct merge_tables;
 
-// Iterations to enqueue before the next completion test: at least `least`,
-// else half of those that the mean convergence so far says are left. A test
-// drains the device (a copy, a wake-up and the next graph launch, about 10 us),
-// and an iteration past the end costs its launches, which return at once.
-int iterations_ahead(int least, double residual, std::int64_t iterations, double tol);
+// Iterations to enqueue before the next completion test: `every` as the caller
+// set it; with the default, at least that many, else half of those that the mean
+// convergence so far says are left, at most 32. A test drains the device (a
+// copy, a wake-up and the next graph launch, about 10 us), and an iteration past
+// the end costs its launches, which return at once.
+int iterations_ahead(int every, double residual, std::int64_t iterations, double tol);
 
 // What a grouped solve (solver_group) needs of one member solver: its device
 // arrays, its solve-state defaults and the steps of its two sweeps (launched

@@ -276,7 +276,7 @@ std::vector<solve_result> solver_group::solve(const std::vector<const double*>& 
         check(hipStreamEndCapture(P.cap, &P.graph), "hipStreamEndCapture");
         check(hipGraphInstantiate(&P.exec, P.graph, nullptr, nullptr, 0), "hipGraphInstantiate");
     }
-    const int J = 2;
+    const int J = kItersPerCheck;
     int enqueued = 0, step = J;
     for (;;) {
         for (int j = 0; j < step; ++j) check(hipGraphLaunch(P.exec, s), "hipGraphLaunch");
