@@ -837,17 +837,26 @@ void gpu_solver::setup(const csc_view& L) {
     // rows in original vertex order (a row map), so a band of slices -- one
     // XCD's share, see spmv_sell -- gathers from a band of vertices and its
     // neighbours; unsorted when 64-row slices pad to <= 1.2 x the entries,
-    // else sorted by length inside 4096-row windows (rows longer than
-    // max(32, mean) walked by a wave) when that pads to <= 1.5 x; otherwise
-    // CSR lanes only. APXCHOL_AMD_SPMV=csr / sell forces the choice;
+    // else sorted by length inside 4096-row windows when that pads to <= 1.5 x;
+    // otherwise CSR lanes only. Long rows are left out and walked by a wave. APXCHOL_AMD_SPMV=csr / sell forces the choice;
     // APXCHOL_AMD_SELL_ORDER=storage slices in storage order instead.
     {
         const std::int64_t nnz = op.ptr.back();
-        // A lane walks its row of a slice alone, a wave the rows past the mean:
-        // the longest lane chain is the launch's critical path (SpMV calls at
-        // max(64, 8 mean) / max(64, 2 mean) / max(32, mean): R-MAT s14 28.9 /
-        // 16.9 / 14.1 us, s18 122 / 79 / 80).
-        const std::int64_t long_len = std::max<std::int64_t>(32, static_cast<std::int64_t>(std::ceil(avg)));
+        // Rows longer than len and their entries.
+        const auto longer = [&](std::int64_t len) {
+            std::pair<std::int64_t, std::int64_t> c{0, 0};
+            for (int r = 0; r < n; ++r) {
+                const std::int64_t q = op.ptr[r + 1] - op.ptr[r];
+                if (q > len) { ++c.first; c.second += q; }
+            }
+            return c;
+        };
+        const std::int64_t mean = static_cast<std::int64_t>(std::ceil(avg));
+        // Whether the slices pad little enough is asked with the hub rows alone
+        // left out: small graphs whose slices only fit without every row past
+        // the mean have too few slices for blocks (R-MAT scale 9, 64 columns:
+        // 100 us, CSR lanes 18).
+        const std::int64_t form_len = std::max<std::int64_t>(64, 8 * mean);
         const char* fe = std::getenv("APXCHOL_AMD_SPMV");
         const std::string force = fe ? fe : "";
         const char* oe = std::getenv("APXCHOL_AMD_SELL_ORDER");
@@ -855,20 +864,26 @@ void gpu_solver::setup(const csc_view& L) {
         if (n > 0 && force != "csr") {
             std::vector<std::int32_t> rows(static_cast<std::size_t>(n));
             for (int v = 0; v < n; ++v) rows[v] = storage_order ? v : static_cast<std::int32_t>(sperm[v]);
-            std::int64_t long_nnz = 0;
-            for (int r = 0; r < n; ++r)
-                if (op.ptr[r + 1] - op.ptr[r] > long_len) long_nnz += op.ptr[r + 1] - op.ptr[r];
-            const double short_nnz = static_cast<double>(std::max<std::int64_t>(nnz - long_nnz, 1));
-            sell_layout sl;
-            bool ok = false;
-            if (static_cast<double>(sell_slots(op, long_len, rows)) <= 1.2 * short_nnz) {
-                sl = build_sell(op, long_len, 1, rows);
-                ok = true;
-            } else {
-                sl = build_sell(op, long_len, 4096, rows);
-                ok = force == "sell" || static_cast<double>(sl.slots) <= 1.5 * short_nnz;
-            }
+            const double form_nnz = static_cast<double>(std::max<std::int64_t>(nnz - longer(form_len).second, 1));
+            const bool ok = force == "sell" || static_cast<double>(sell_slots(op, form_len, rows)) <= 1.2 * form_nnz ||
+                            static_cast<double>(sell_slots(op, form_len, rows, 4096)) <= 1.5 * form_nnz;
             if (ok) {
+                // A lane walks its row of a slice alone, a wave the long rows:
+                // the longest lane chain is the launch's critical path (SpMV
+                // calls at max(64, 8 mean) / max(64, 2 mean) / max(32, mean):
+                // R-MAT s14 28.9 / 16.9 / 14.1 us, s18 122 / 79 / 80; of a
+                // power-law graph 10 to 25 % of the rows pass the mean). Where
+                // more do they are no tail, and slices are the better form
+                // (past the mean / past twice the mean: random graph of 50,000
+                // vertices, 41 entries a row, SpMV 49 / 34 us, 32 columns 176 /
+                // 114; 5^3-point stencil on 40^3, 4 columns 88 / 46, 32 columns
+                // 460 / 205; only small single products lose, 5,000 vertices
+                // 16 / 25).
+                std::int64_t long_len = std::max<std::int64_t>(32, mean);
+                if (4 * longer(long_len).first > n) long_len = std::max<std::int64_t>(64, 2 * mean);
+                const double short_nnz = static_cast<double>(std::max<std::int64_t>(nnz - longer(long_len).second, 1));
+                const bool unsorted = static_cast<double>(sell_slots(op, long_len, rows)) <= 1.2 * short_nnz;
+                const sell_layout sl = build_sell(op, long_len, unsorted ? 1 : 4096, rows);
                 d.sell_soff.upload(sl.soff);
                 d.sell_idx.upload(sl.idx);
                 if (d.op32) d.sell_val.upload(sl.val32); else d.sell_val.upload(sl.val);

@@ -24,8 +24,9 @@ namespace {
 // lose 4 %, at four times it as well.
 constexpr double kLaunchUs = 3.6, kLevelUs = 0.8, kTileBatchUs = 0.11, kBatchUs = 0.001;
 constexpr int kUnits = 256;   // compute units
-// Tiles a trial looks at (128^3: a solve 25.4 ms; with all 25.2 and 40 ms more
-// of host time, with 4 26.0 and as much time).
+// Tiles a trial looks at. A mixed 128^3 solve and the host time of its tiles
+// (the trials one after another and the tables in one array): all 25.2 ms and
+// 0.17 s, 32 25.4 and 0.13, 4 26.0 and 0.13.
 constexpr int kSampleTiles = 32;
 
 double launch_us(int levels, double batches, double tile_batches) {

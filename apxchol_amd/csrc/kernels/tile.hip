@@ -12,8 +12,9 @@
 // shared rows allow it: with 16 a compute unit's gathers, a line a cycle, are
 // the longest part (four levels of a 256^2 grid: 8.9 us, with 4 waves 6.7, as
 // launches of their own 4 x 3.9).
-// Solves: 256^2 fp64 6,880 -> 5,900 us, 128^3 SDDM mixed 28,700 -> 25,600 (148
-// -> 82 launched levels an iteration), R-MAT scale 18 mixed 6,750 -> 6,000.
+// Solves without and with tiles: 256^2 fp64 7,180 / 6,060 us, 128^3 SDDM mixed
+// 28,600 / 25,500 (148 / 86 launched levels an iteration), R-MAT scale 18 mixed
+// 7,180 / 6,480 (60 / 43).
 namespace apxchol_amd {
 
 inline constexpr int kTileBlock = kTileWaves * kWave;

@@ -3,7 +3,7 @@
 //
 // The last eliminations of an approximate Cholesky factor are its long, thin
 // part: on an 89^3 grid 129 of the 169 dependent levels of a sweep hold 4,832
-// of 704,969 rows, on an R-MAT graph of scale 18 1,930 of 1,964 hold 6,000 of
+// of 704,969 rows, on an R-MAT graph of scale 18 1,934 of 1,964 hold 7,004 of
 // 262,143. Walking them costs a launch or a barrier per level and direction
 // (0.6 .. 4.5 us each) for almost no bytes. With the rows split as P (before
 // the block) and T (the block), L = [L_PP 0; L_TP T_], the pair of sweeps is
@@ -24,8 +24,9 @@
 // application against fp64: walked 8.5e-7, fp32 sums 1.5e-6, fp64 sums 3.9e-7;
 // the product stays bound by its bytes).
 //
-// The block's first row depends on the factor and the vector precision alone,
-// never on the schedule, and the kernels below give every column of a block
+// The block's first row depends on the factor and the vector precision alone
+// (there is none where device memory does not suffice), never on the schedule,
+// and the kernels below give every column of a block
 // and every member of a group the single application's arithmetic, so all
 // schedules keep agreeing bit for bit.
 #include "common.hpp"
@@ -133,9 +134,9 @@ __device__ __forceinline__ double trail_skip(TO v, double c, double acc) {
 }
 __device__ __forceinline__ bool trail_finite(double v) { return fabs(v) <= 1.7976931348623157e308; }
 
-// z_T = S c. HBM-bound: S is read once, n^2 values (R-MAT s18, 6,006 fp32
-// rows, 144 MB: 28.7 us, 5.0 TB/s, the rate of a plain copy; 256^2 grid, 1,551
-// fp64 rows, 19 MB: 8 us). With the coupling launch (31.6 us there: hub rows)
+// z_T = S c. HBM-bound: S is read once, n^2 values (R-MAT s18, 7,004 fp32 rows,
+// 196 MB: 35.2 us, 5.6 TB/s; 48^3 grid, 3,773 fp64 rows, 114 MB: 20.1 us, 5.7
+// TB/s; a plain copy moves 5.0). With the coupling launch (35.0 us there: hub rows)
 // it replaces 12 tail runs of 115 us and their couplings an iteration. A workgroup of 16 waves
 // owns kTrailLine / sizeof(TO) rows (one 128-byte line of every row of S,
 // which is symmetric, so a row is read as a column) and cuts the sum over k
