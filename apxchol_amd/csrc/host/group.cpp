@@ -67,6 +67,7 @@ struct solver_group::impl {
     // Stage 2 of the reductions left to their consumers (every member's
     // partials few enough).
     bool fuse_pAp = false, fuse_dot = false;
+    bool long_rows = false;      // of some member's operator
     // One sweep step: its level units, then its tail units, in units[dir].
     struct step {
         int lv_off = 0, lv_count = 0, lv_s = 0, lv_blocks = 0;
@@ -115,7 +116,7 @@ struct solver_group::impl {
     }
     // One PCG iteration of every member (gpu_solver::enqueue_iteration).
     void iteration(hipStream_t s) const {
-        launch_group_spmv(M(), S(spmv_s), count, spmv_blocks, s);
+        launch_group_spmv(M(), S(spmv_s), count, spmv_blocks, long_rows, s);
         if (!fuse_pAp) launch_group_finish(group_fin_op("pAp"), M(), S(spmv_s), count, 0, s);
         launch_group_update_xr(prec, M(), S(vec_s), count, vec_blocks, fuse_pAp ? S(spmv_s) : nullptr, s);
         launch_group_finish(group_fin_op("xr"), M(), S(vec_s), count, fuse_pAp ? kFusedPartOffset : 0, s);
@@ -153,6 +154,7 @@ solver_group::solver_group(std::vector<std::shared_ptr<const gpu_solver>> member
         g.st = st + i;
         mem.push_back(g);
         g_spmv.push_back(group_spmv_blocks(g));
+        P.long_rows = P.long_rows || (g.use_sell && g.sell.nlong > 0);
         g_vec.push_back(group_vec_blocks(g.n));
     }
     P.mem.upload(mem);

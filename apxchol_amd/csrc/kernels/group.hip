@@ -40,6 +40,9 @@ __device__ __forceinline__ void group_spmv_csr(int vb, int vg, const group_membe
 }
 
 // Ap = A p and the partials of p.Ap, every member with its own SpMV form.
+// LONG: some member has long rows, whose walk takes 160 registers (three waves a
+// SIMD instead of eight: 16 SDDM grids of 40^3 12.2 -> 12.7 ms a solve).
+template <bool LONG>
 __global__ __launch_bounds__(kBlock) void group_spmv(const group_member* __restrict__ mem,
                                                      const int* __restrict__ starts, int count) {
     const int b = static_cast<int>(blockIdx.x);
@@ -47,7 +50,7 @@ __global__ __launch_bounds__(kBlock) void group_spmv(const group_member* __restr
     const group_member& g = mem[i];
     const int vb = b - starts[i], vg = starts[i + 1] - starts[i];
     if (g.use_sell) {
-        if (g.sell.nlong > 0) {
+        if (LONG && g.sell.nlong > 0) {
             if (g.val32) spmv_sell_body<float, true>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
             else spmv_sell_body<double, true>(vb, vg, g.sell, g.p, g.ap, g.st, g.part, 1);
         } else {

@@ -1060,9 +1060,11 @@ int group_fin_op(const char* name) {
     throw std::invalid_argument("apxchol_amd: unknown reduction stage " + k);
 }
 
-void launch_group_spmv(const group_member* mem, const int* starts, int count, int blocks, hipStream_t s) {
+void launch_group_spmv(const group_member* mem, const int* starts, int count, int blocks, bool long_rows,
+                       hipStream_t s) {
     if (count <= 0 || blocks <= 0) return;
-    group_spmv<<<blocks, kBlock, 0, s>>>(mem, starts, count);
+    if (long_rows) group_spmv<true><<<blocks, kBlock, 0, s>>>(mem, starts, count);
+    else group_spmv<false><<<blocks, kBlock, 0, s>>>(mem, starts, count);
     check_launch("group_spmv");
 }
 

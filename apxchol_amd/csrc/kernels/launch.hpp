@@ -296,7 +296,9 @@ struct group_unit {
 // The own grid of a member's single-vector SpMV and of its vector passes.
 int group_spmv_blocks(const group_member& g);
 int group_vec_blocks(int n);
-void launch_group_spmv(const group_member* mem, const int* starts, int count, int blocks, hipStream_t s);
+// long_rows: some member's sliced-ELL form has rows outside its slices.
+void launch_group_spmv(const group_member* mem, const int* starts, int count, int blocks, bool long_rows,
+                       hipStream_t s);
 // offset: where the members' partials start in their buffers.
 void launch_group_finish(int op, const group_member* mem, const int* starts, int count, int offset, hipStream_t s);
 // dot_starts: the SpMV's starts when stage 2 of its reduction is left to this
