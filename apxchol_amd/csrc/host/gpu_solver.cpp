@@ -1007,6 +1007,38 @@ void gpu_solver::setup(const csc_view& L) {
         }
         if (!formed) cut = L_all;
     }
+    // An application's steps outside the trailing block, the two directions side
+    // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
+    // may gain; 0: no merging).
+    long long growth = opts_.merge_levels ? -1 : 0;
+    if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
+    // (Of 1024 levels and more outside the block most are small: not tried.)
+    bool merging = d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0 && (growth > 0 || cut < 1024);
+    merge_tables mt[2];
+    if (merging) {
+        const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
+        side_by_side(2, [&](int dir) {
+            mt[dir] = dir ? build_merged_levels(T_, true, L - c, L, d.b_levels, growth)
+                          : build_merged_levels(T_, false, 0, c, d.f_levels, growth);
+        });
+        // Merged levels have no tail runs, which walk a small level in a quarter
+        // of a launch: a long chain of them outside the block (R-MAT scale 22:
+        // ~6,000 levels) is faster walked (fp64 solve 773 ms merged). By the
+        // factor alone, so that every schedule agrees on it.
+        double walked = 0;
+        for (int q = 0; q < c; ++q) walked += d.f_levels[q + 1] - d.f_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
+        for (int q = L - c; q < L; ++q) walked += d.b_levels[q + 1] - d.b_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
+        merging = growth > 0 || 4.5 * static_cast<double>(mt[0].steps.size() + mt[1].steps.size()) < walked;
+    }
+    if (merging) {
+        try {
+            upload_merged(mt[0], mt[1]);
+        } catch (const device_memory_error&) {
+            merging = false;
+            for (int dir = 0; dir < 2; ++dir)
+                for (dbuf* b : {&d.mg_rec[dir], &d.mg_batch[dir], &d.mg_idx[dir], &d.mg_val[dir]}) b->alloc(0);
+        }
+    }
     // What the level tiles of a direction are built from.
     struct tile_input {
         lane_tables lt;
@@ -1051,8 +1083,10 @@ void gpu_solver::setup(const csc_view& L) {
             }
             return worst;
         };
-        // The trailing block's boundary in this direction; no run crosses it.
+        // The trailing block's boundary in this direction; no run crosses it
+        // unless applications follow the merged levels instead of these runs.
         const int cl = backward ? L - static_cast<int>(cut) : static_cast<int>(cut);
+        const int stop = merging ? -1 : cl;
         sc.cut_level = cl;
         sc.cut_batch = lf[cl];
         for (int l = 0; l < L;) {
@@ -1064,7 +1098,7 @@ void gpu_solver::setup(const csc_view& L) {
                 continue;
             }
             int e = l;
-            while (e < L && (e == l || e != cl) && small(e) && sweep_tail_fits(tail_prec, pos(e + 1) - pos(l), lf[e + 1] - lf[l], e + 1 - l) &&
+            while (e < L && (e == l || e != stop) && small(e) && sweep_tail_fits(tail_prec, pos(e + 1) - pos(l), lf[e + 1] - lf[l], e + 1 - l) &&
                    (e == l || tail_cut <= 0 || ovf_groups(e, pos(l)) < tail_cut))
                 ++e;
             if (e == l) ++e;   // a single small level always fits (rows < tail_rows <= cap)
@@ -1114,7 +1148,7 @@ void gpu_solver::setup(const csc_view& L) {
                 static_cast<std::uint64_t>(std::max(env_flag("APXCHOL_AMD_COUPLE_SPLIT_MIN", 1 << 20), 0));
             for (std::size_t k = 1; k < seg[0].size(); ++k) {
                 if (!seg[2][k] || !seg[2][k - 1] || seg[3][k - 1] <= 0) continue;
-                if (static_cast<int>(k) == sc.cut_seg) continue;   // a launch may start here
+                if (!merging && static_cast<int>(k) == sc.cut_seg) continue;   // a launch may start here
                 const int ps = seg[3][k - 1];
                 std::uint64_t before = 0;
                 for (int t = seg[3][k]; t < seg[4][k]; ++t) {
@@ -1262,38 +1296,7 @@ void gpu_solver::setup(const csc_view& L) {
                d.f_level_pos, d.f_level_diag);
     make_sched(d.b_sched, bb, true, d.b_levels, d.b_levels_dev, d.b_seg, b_tb, d.b_level_lb, d.b_lrec, d.b_lent,
                d.b_level_pos, d.b_level_diag);
-    // An application's steps outside the trailing block, the two directions side
-    // by side (fp64 vectors; APXCHOL_AMD_MERGE_GROWTH: entries a merged level
-    // may gain; 0: no merging).
-    long long growth = opts_.merge_levels ? -1 : 0;
-    if (const char* e = std::getenv("APXCHOL_AMD_MERGE_GROWTH"); e && *e) growth = std::max(0, std::atoi(e));
-    // (Of 1024 levels and more outside the block most are small: not tried.)
-    bool merging = d.trail.n > 0 && d.prec == vec_prec::fp64 && growth != 0 && (growth > 0 || cut < 1024);
-    merge_tables mt[2];
-    if (merging) {
-        const int L = static_cast<int>(L_all), c = static_cast<int>(cut);
-        side_by_side(2, [&](int dir) {
-            mt[dir] = dir ? build_merged_levels(T_, true, L - c, L, d.b_levels, growth)
-                          : build_merged_levels(T_, false, 0, c, d.f_levels, growth);
-        });
-        // Merged levels have no tail runs, which walk a small level in a quarter
-        // of a launch: a long chain of them outside the block (R-MAT scale 22:
-        // ~6,000 levels) is faster walked (fp64 solve 773 ms merged). By the
-        // factor alone, so that every schedule agrees on it.
-        double walked = 0;
-        for (int q = 0; q < c; ++q) walked += d.f_levels[q + 1] - d.f_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
-        for (int q = L - c; q < L; ++q) walked += d.b_levels[q + 1] - d.b_levels[q] > 3 * kTailWaves ? 4.1 : 1.0;
-        merging = growth > 0 || 4.5 * static_cast<double>(mt[0].steps.size() + mt[1].steps.size()) < walked;
-    }
-    if (merging) {
-        try {
-            upload_merged(mt[0], mt[1]);
-        } catch (const device_memory_error&) {
-            merging = false;
-            for (int dir = 0; dir < 2; ++dir)
-                for (dbuf* b : {&d.mg_rec[dir], &d.mg_batch[dir], &d.mg_idx[dir], &d.mg_val[dir]}) b->alloc(0);
-        }
-    }
+    if (merging) follow_merged(mt[0], mt[1]);
     // Level tiles, the two directions side by side, where levels are not merged
     // (APXCHOL_AMD_TILE_LEVELS: levels a launch may join, 1: none). A solver for
     // one solve goes without: on a mixed 128^3 system they take 80 ms and save
@@ -1423,6 +1426,10 @@ void gpu_solver::upload_merged(const merge_tables& fwd, const merge_tables& bck)
             at += q.idx.size();
         }
     }
+}
+
+void gpu_solver::follow_merged(const merge_tables& fwd, const merge_tables& bck) {
+    auto& d = *dev_;
     for (int dir = 0; dir < 2; ++dir) {
         const merge_tables& t = dir ? bck : fwd;
         d.plan[dir] = t.steps;

@@ -281,8 +281,9 @@ private:
     // block) when its inverse leaves the vectors' range or its rounding could
     // spoil it (trail_is_sound).
     bool build_trail(std::uint32_t first);
-    // Makes applications follow the merged levels.
+    // Uploads the merged levels; makes applications follow them.
     void upload_merged(const merge_tables& fwd, const merge_tables& bck);
+    void follow_merged(const merge_tables& fwd, const merge_tables& bck);
     // z = (L L^T)^-1 r in storage order: the forward levels, the trailing
     // block, the back levels; one vector, and kp columns of block `which`.
     void enqueue_pair(const double* r, const pcg_state* st, int step, hipStream_t s) const;
