@@ -237,21 +237,12 @@ __global__ __launch_bounds__(kTrailThreads) void trail_apply_k(trail_desc t, con
     constexpr int kPerWave = kChunks / kTrailWaves;
     static_assert(kTrailWaves * kWave * CT * sizeof(double) <= 65536, "static LDS");
     __shared__ double red[kTrailWaves][CT][kWave];
-    const int lane = threadIdx.x & (kWave - 1);
-    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
-    const int i = static_cast<int>(blockIdx.x) * kWave + lane;   // < ld: rows past n are zero in S
     const int c0 = static_cast<int>(blockIdx.y) * CT;
-    // Output o of this workgroup is row blockIdx.x * kWave + o % kWave of column
-    // c0 + o / kWave; this thread's are every kTrailThreads-th.
-    constexpr int kOut = (kWave * CT + kTrailThreads - 1) / kTrailThreads;
-    double sum[kOut];
-    const auto row_of = [&](int x) {
-        const int o = static_cast<int>(threadIdx.x) + x * kTrailThreads;
-        const int row = static_cast<int>(blockIdx.x) * kWave + (o & (kWave - 1));
-        return o < kWave * CT && row < t.n ? row : -1;
-    };
-    // Returns whether every sum of this thread is finite.
-    const auto product = [&](auto skip_zeros) {
+    // Returns whether every output of this thread is finite.
+    const auto product = [&](auto skip_zeros, int tid) {
+        const int lane = tid & (kWave - 1);
+        const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+        const int i = static_cast<int>(blockIdx.x) * kWave + lane;   // < ld: rows past n are zero in S
         double q[CT];
 #pragma unroll
         for (int j = 0; j < kPerWave; ++j) {
@@ -295,28 +286,26 @@ __global__ __launch_bounds__(kTrailThreads) void trail_apply_k(trail_desc t, con
         for (int u = 0; u < CT; ++u) red[w][u][lane] = q[u];
         __syncthreads();
         bool finite = true;
+        for (int o = tid; o < kWave * CT; o += kTrailThreads) {
+            const int rl = o & (kWave - 1), u = o / kWave;
+            const int row = static_cast<int>(blockIdx.x) * kWave + rl;
+            if (row >= t.n) continue;
+            double sum = red[0][u][rl];
 #pragma unroll
-        for (int x = 0; x < kOut; ++x) {
-            sum[x] = 0.0;
-            if (row_of(x) < 0) continue;
-            const int o = static_cast<int>(threadIdx.x) + x * kTrailThreads, rl = o & (kWave - 1), u = o / kWave;
-            sum[x] = red[0][u][rl];
-#pragma unroll
-            for (int v = 1; v < kTrailWaves; ++v) sum[x] += red[v][u][rl];
-            finite = finite && trail_finite(sum[x]);
+            for (int v = 1; v < kTrailWaves; ++v) sum += red[v][u][rl];
+            z[static_cast<size_t>(t.first + row) * kp + c0 + u] = static_cast<TO>(sum);
+            finite = finite && trail_finite(sum);
         }
         return finite;
     };
+    int tid = static_cast<int>(threadIdx.x);
     __shared__ int again;
-    if (threadIdx.x == 0) again = 0;   // (a barrier of the product follows)
-    if (!product(std::false_type{})) again = 1;
+    if (tid == 0) again = 0;   // (a barrier of the product follows)
+    if (!product(std::false_type{}, tid)) again = 1;
     __syncthreads();
-    if (again) (void)product(std::true_type{});
-#pragma unroll
-    for (int x = 0; x < kOut; ++x) {
-        if (row_of(x) < 0) continue;
-        const int u = (static_cast<int>(threadIdx.x) + x * kTrailThreads) / kWave;
-        z[static_cast<size_t>(t.first + row_of(x)) * kp + c0 + u] = static_cast<TO>(sum[x]);
+    if (again) {
+        asm volatile("" : "+v"(tid));   // nothing of the first pass is kept for this one
+        (void)product(std::true_type{}, tid);
     }
 }
 
