@@ -38,7 +38,10 @@ typedef struct {
     int32_t precision;       /* sweep vectors: 0 = fp64, 1 = fp32 (factor values are fp32 or fp16) */
     int32_t fp16_storage;    /* 1 = per-column-scaled fp16 factor values */
     int32_t schedule;        /* 0 = sync-free dataflow, 1 = level-set launches, 2 = hybrid (default):
-                                big levels launched, runs of small levels walked by one workgroup */
+                                big levels launched, runs of small levels walked by one workgroup.
+                                Applications of a factor with merged levels (precision 0 with a
+                                trailing block) follow their own steps; this and the tail options
+                                then act on whole sweeps (apx_solver_sweep) only */
     double drop_rel;         /* < 0: APXCHOL_FACTOR_DROP or 1e-4; 0 disables the drop */
     int32_t keep_factor;     /* keep the host factor values for apx_solver_export_factor */
     int32_t iters_per_check; /* PCG iterations enqueued between completion tests; 2 (default, and 0):
@@ -152,7 +155,8 @@ void apx_solver_destroy(apx_solver_t s);
 apx_status apx_solver_info_get(apx_solver_t s, apx_solver_info* info);
 
 /* What one preconditioner application runs. The last `rows` rows of the factor
- * (0: none) are applied through their explicit inverse, `bytes` of it, by one
+ * (0: none -- a thin factor, one too soft for an explicit inverse, or no memory
+ * for it) are applied through their explicit inverse, `bytes` of it, by one
  * coupling launch and one matrix-vector product; the levels before them as
  * apx_solver_info describes whole sweeps: per direction [0 forward, 1 back]
  * the bytes and counts of the level launches and tail runs outside the block. */
